@@ -33,6 +33,7 @@
 #include "kve_gemm.h"
 
 #include <algorithm>
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
@@ -1050,8 +1051,8 @@ __global__ __launch_bounds__(C::NT) void gate_up_silu_kernel(const uint16_t* xn,
 // state do not depend on which pass computed them. linear_splitk_kernel
 // computes, per output element, one MFMA chain per k-slice (from zero, k-steps
 // in order) and its reductions add the slices in order; gate_up_silu_kernel
-// runs one chain over all of K. Here a workgroup takes 128 weight rows x 128
-// rows over the whole of K and keeps both sums in registers: acc is the
+// runs one chain over all of K. Here a workgroup takes 128 weight rows x up
+// to 256 rows over the whole of K and keeps both sums in registers: acc is the
 // current slice's chain, added to tot and restarted at every slice boundary.
 // MODE 0: tot starts at -0, the additive identity, so it ends as
 // t0 + t1 + ... (residual_norm_kernel's acc = t0, acc += t1, ...); MODE 1: at
@@ -1063,76 +1064,183 @@ __global__ __launch_bounds__(C::NT) void gate_up_silu_kernel(const uint16_t* xn,
 // The chains use the same MFMA with the same operands per lane (weight rows
 // on the A side, 8 consecutive k of a k-step per lane group), so each slice
 // sum is the split-K kernel's bit for bit.
-template <int MT_, int NW_, int WN_, int KC_, int LDS_, int NR_>
+//
+// Tile and pipeline. 4 waves as 2 x 2 groups of 64 weight rows x 16 MTW rows: a
+// 128 x 32 MTW tile in at most 80 KB of LDS and 256 registers, so two
+// workgroups share a CU and one multiplies while the other waits at its
+// barrier, loads its first k-steps or writes its outputs. Each k-step has its
+// own LDS buffer (NB of them, NB - 1 in flight): 16-row x 32-column pieces of
+// 1 KB, one per direct load, their 16-byte units swizzled so the 16 rows of a
+// fragment read fall in different bank groups. A k-step's fragments are read,
+// and a later k-step's loads issued, in between the previous k-step's MFMAs
+// (the scheduling barriers hold every read and load at its place): one barrier
+// per k-step, no LDS latency in front of the MFMAs. Workgroups are dealt to the
+// XCDs in contiguous runs of tiles, 4 row tiles by columns, so the 64 tiles an
+// XCD has in flight share their operands in its L2.
+// Before: a 128 x 256 tile on 16 waves (32 x 64 each), one workgroup per CU,
+// fragments read at the start of each chunk, tiles in launch order. It was
+// bound by LDS (192 bytes of fragments per clock at full MFMA rate, 128 are
+// served) and by the chunk waits that every wave of the CU shared. 3B layer at
+// 6154 rows, us and TFLOP/s, before -> now: gate/up 664 -> 474 (836 -> 1170),
+// down 332 -> 261 (836 -> 1064), o 81 -> 63 (637 -> 823); at 3000 rows 338 ->
+// 232, 177 -> 134, 65 -> 33. Measured beside it: a 256 x 256 tile on 8 waves
+// (gate/up 471-497 us at 6154 rows) or on 4 (484-506), one workgroup per CU.
+template <int MTW_, int NB_>
 struct RowsTile {
-  using G = typename DmaCfg<MT_, NW_, WN_, KC_, LDS_, NR_>::G;
-  static constexpr int NT = 64 * NW_;
+  static constexpr int WN = 4, MTW = MTW_, NC = 2, NR = 2, NW = NC * NR, NT = 64 * NW, NB = NB_;
+  static constexpr int BN = 16 * WN * NC, BM = 16 * MTW * NR;
+  static constexpr int PIECES = (BN + BM) / 16;      // 1 KB pieces of a k-step
+  static constexpr int U = cdiv(PIECES, NW);         // of which each wave loads U
+  static constexpr int BUF = PIECES * 512;           // elements of a k-step's buffer
+  static constexpr size_t LDS = static_cast<size_t>(NB) * BUF * 2;
 };
-// 16 waves (four per SIMD) as 4 column x 4 row groups, each 32 weight rows x
-// 64 rows: a 128 x 256 tile, three 48 KB chunk buffers. Measured on the 3B layer
-// at 5400 rows, 8 waves with 128 x 256 tiles against 4 waves with 128 x 128:
-// 2.19 -> 1.24 ms; 16 waves against 8 (the same tile, more waves issuing the
-// chunk loads) at 4096 rows: q/k/v 89.5 -> 80.4 us, o 52.4 -> 47.5, gate/up
-// 529 -> 490, down 209 -> 195 (535 / 722 / 754 / 948 TFLOP/s); one-k-step
-// chunks with five in flight measured slower on 8 and on 16 waves.
-using RowsCfg = RowsTile<16, 16, 2, 2, 144 * 1024, 4>;
 
-template <int MODE, bool SLICED, typename C, bool BLK = false>
-__global__ __launch_bounds__(C::NT) void linear_rows_kernel(const uint16_t* x, const uint16_t* w,
-                                                            void* out, int M, int N, int K, int S) {
-  using G = typename C::G;
-  constexpr int WN = G::BN / (16 * G::NC), MTW = G::MTW, BM = G::XROWS, HALF = WN / 2;
-  static_assert(WN % 2 == 0, "gate and up tiles pair up");
+// MODE 0-2 as above, or kRowsSlice (one k-slice per workgroup, blockIdx.y, written
+// as linear_splitk_kernel writes it). tot is kept only where slices are summed.
+constexpr int kRowsSlice = 3;
+
+template <int MODE, typename C, bool BLK>
+__global__ __launch_bounds__(C::NT, 2) void linear_rows_kernel(const uint16_t* x, const uint16_t* w,
+                                                               void* out, int M, int N, int K, int S,
+                                                               int nx, int ny) {
+  constexpr int WN = C::WN, MTW = C::MTW, HALF = WN / 2, U = C::U, NW = C::NW, NB = C::NB;
+  constexpr int BN = C::BN, BUF = C::BUF;
+  constexpr bool TOT = MODE < 2;
   extern __shared__ __align__(16) uint16_t sm_lin[];
-  const int tid = threadIdx.x;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wc = wv % G::NC, wr = wv / G::NC;
-  const int l = tid & 63, lr = l & 15, lg = l >> 4;
-  const int m0 = blockIdx.y * BM;
-  const int Mb = min(BM, M - m0);
-  const int nks = K / 32;
-  f32x4 acc[WN][MTW], tot[WN][MTW];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wc = wv % C::NC, wr = wv / C::NC;
+  const int l = threadIdx.x & 63, lr = l & 15, lg = l >> 4;
+  // tile (bx, by): XCD L % 8 takes a contiguous run of the tiles, ordered as
+  // bands of GY row tiles, column by column within a band
+  constexpr int GY = 4;
+  int bx, by;
+  {
+    const int n = nx * ny, q = n / 8, r = n % 8, xcd = blockIdx.x % 8;
+    const int t = xcd * q + min(xcd, r) + static_cast<int>(blockIdx.x) / 8;
+    const int band = t / (GY * nx), y0 = band * GY, h = min(GY, ny - y0), o = t - band * GY * nx;
+    by = y0 + o % h;
+    bx = o / h;
+  }
+  const int m0 = by * C::BM, Mb = min(C::BM, M - m0);
+  const int f0 = bx * (BN / 2), n0 = bx * BN, F = N;  // MODE 2: N is the activation width
+  int ka = 0, kb = K / 32;                            // k-steps of this workgroup
+  if (MODE == kRowsSlice) split_range(K / 32, S, blockIdx.y, ka, kb);
+
+  // this wave's pieces NW i + wv (the last one again past PIECES: same bytes to
+  // the same place): lane l fills 16-byte unit l, which holds unit c of row r
+  const uint16_t* src[U];
+#pragma unroll
+  for (int i = 0; i < U; ++i) {
+    const int t = min(NW * i + wv, C::PIECES - 1);
+    const int r = l >> 2, c = (l & 3) ^ ((r >> 2) & 3);
+    int row;
+    if (t >= BN / 16) {
+      row = m0 + min(16 * (t - BN / 16) + r, Mb - 1);
+    } else if (MODE == 2) {
+      const int j = t % WN, col = f0 + 16 * (HALF * (t / WN) + j % HALF) + r;
+      row = j < HALF ? col : F + col;
+    } else {
+      row = n0 + 16 * t + r;
+    }
+    src[i] = (t < BN / 16 ? w : x) + mat_off(row, 8 * c, K, K, BLK);
+  }
+  constexpr int KSTEP = BLK ? 512 : 32;  // elements from one k-step to the next
+  auto dma = [&](int i, int ks, uint16_t* buf) {
+    __builtin_amdgcn_global_load_lds(
+        (__attribute__((address_space(1))) void*)(src[i] + KSTEP * ks),
+        (__attribute__((address_space(3))) void*)(buf + 512 * min(NW * i + wv, C::PIECES - 1)), 16, 0,
+        0);
+  };
+  auto rd = [](const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); };
+  const int fo = 8 * (lr * 4 + (lg ^ ((lr >> 2) & 3)));
+  const int ao = WN * wc * 512 + fo, bo = (BN / 16 + MTW * wr) * 512 + fo;
+
+  f32x4 acc[WN][MTW], tot[TOT ? WN : 1][TOT ? MTW : 1];
   const float t0 = MODE == 1 ? 0.0f : -0.0f;
 #pragma unroll
   for (int j = 0; j < WN; ++j)
 #pragma unroll
     for (int mt = 0; mt < MTW; ++mt) {
       acc[j][mt] = f32x4{0, 0, 0, 0};
-      tot[j][mt] = f32x4{t0, t0, t0, t0};
+      if constexpr (TOT) tot[j][mt] = f32x4{t0, t0, t0, t0};
     }
-  int s = 0, next = nks / S;  // end of slice 0 (split_range)
-  auto fold = [&](int ks) {
-    if (ks + 1 != next) return;
+  // Every load is issued (k-steps past kb re-read the last one into buffers
+  // nothing reads), so each wait below is exact.
 #pragma unroll
-    for (int j = 0; j < WN; ++j)
+  for (int q = 0; q < NB - 1; ++q)
 #pragma unroll
-      for (int mt = 0; mt < MTW; ++mt) {
-        tot[j][mt] += acc[j][mt];
-        acc[j][mt] = f32x4{0, 0, 0, 0};
+    for (int i = 0; i < U; ++i) dma(i, min(ka + q, kb - 1), sm_lin + q * BUF);
+  barrier_after_vm<(NB - 2) * U>();
+  u32x4 fa[2][WN], fb[2][MTW];
+#pragma unroll
+  for (int j = 0; j < WN; ++j) fa[0][j] = rd(sm_lin + ao + 512 * j);
+#pragma unroll
+  for (int mt = 0; mt < MTW; ++mt) fb[0][mt] = rd(sm_lin + bo + 512 * mt);
+#pragma unroll
+  for (int i = 0; i < U; ++i) dma(i, min(ka + NB - 1, kb - 1), sm_lin + (NB - 1) * BUF);
+
+  int s = 0, next = TOT ? kb / S : 0;  // end of slice 0 (split_range)
+  auto step = [&](int ks, auto CUR) {
+    constexpr int cur = decltype(CUR)::value, nxt = cur ^ 1;
+    // k-step ks + 1 has landed for every wave, and every wave has read its
+    // fragments of ks, whose buffer takes k-step ks + NB
+    barrier_after_vm<(NB - 2) * U>();
+    const uint16_t* nb = sm_lin + ((ks - ka + 1) % NB) * BUF;
+    uint16_t* db = sm_lin + ((ks - ka) % NB) * BUF;
+    const int dk = min(ks + NB, kb - 1);
+    // SLOTS fragment reads and loads, evenly over the first 85 % of the MFMAs
+    constexpr int MF = WN * MTW, SLOTS = WN + MTW + U;
+    auto slot = [&](int o) {
+      const int a = o * U / SLOTS;  // loads before this slot
+      if ((o + 1) * U / SLOTS > a) dma(a, dk, db);
+      else if (o - a < MTW) fb[nxt][o - a] = rd(nb + bo + 512 * (o - a));
+      else fa[nxt][o - a - MTW] = rd(nb + ao + 512 * (o - a - MTW));
+    };
+    int o = 0;
+#pragma unroll
+    for (int q = 0; q < MF; ++q) {
+      const int j = q / MTW, mt = q % MTW;
+      acc[j][mt] = mfma16x16x32_bf16(fa[cur][j], fb[cur][mt], acc[j][mt]);
+      const int want = min(SLOTS, (q + 1) * SLOTS * 100 / (MF * 85));
+      if (o < want) {
+        __builtin_amdgcn_sched_barrier(0);
+        for (; o < want; ++o) slot(o);
+        __builtin_amdgcn_sched_barrier(0);
       }
-    ++s;
-    next = static_cast<int>(static_cast<int64_t>(nks) * (s + 1) / S);
-  };
-  const uint16_t* xb = x + static_cast<size_t>(m0) * K;  // row m0 in either layout (m0 % 16 == 0)
-  if (MODE == 2) {
-    const int f0 = blockIdx.x * (G::BN / 2), F = N;
-    G::template run<BLK>(w,
-           [f0, F](int r) {
-             const int t = r >> 4, j = t % WN;
-             const int c = f0 + 16 * (HALF * (t / WN) + j % HALF) + (r & 15);
-             return j < HALF ? c : F + c;
-           },
-           xb, K, Mb, K, 0, nks, sm_lin, acc, fold);
+    }
+    if constexpr (TOT) {
+      if (ks + 1 == next) {
 #pragma unroll
-    for (int mt = 0; mt < MTW; ++mt) {
-      const int m = 16 * (MTW * wr + mt) + lr;
-      if (m >= Mb) continue;
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+          for (int mt = 0; mt < MTW; ++mt) {
+            tot[j][mt] += acc[j][mt];
+            acc[j][mt] = f32x4{0, 0, 0, 0};
+          }
+        ++s;
+        next = static_cast<int>(static_cast<int64_t>(kb) * (s + 1) / S);
+      }
+    }
+  };
+  int ks = ka;
+  for (; ks + 1 < kb; ks += 2) {
+    step(ks, std::integral_constant<int, 0>{});
+    step(ks + 1, std::integral_constant<int, 1>{});
+  }
+  if (ks < kb) step(ks, std::integral_constant<int, 0>{});
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));  // no load may land after the wave has ended
+
+#pragma unroll
+  for (int mt = 0; mt < MTW; ++mt) {
+    const int m = 16 * (MTW * wr + mt) + lr;
+    if (m >= Mb) continue;
+    if constexpr (MODE == 2) {
 #pragma unroll
       for (int j = 0; j < HALF; ++j) {
         float o[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float g = rbf(tot[j][mt][i]), u = rbf(tot[j + HALF][mt][i]);
+          const float g = rbf(acc[j][mt][i]), u = rbf(acc[j + HALF][mt][i]);
           const float sg = rbf(__fdiv_rn(g, __fadd_rn(1.0f, expf(-g))));
           o[i] = __fmul_rn(sg, u);
         }
@@ -1140,34 +1248,14 @@ __global__ __launch_bounds__(C::NT) void linear_rows_kernel(const uint16_t* x, c
         *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(out) + mat_off(m0 + m, c, F, F, BLK)) =
             u32x2{bf_pack(o[0], o[1]), bf_pack(o[2], o[3])};
       }
-    }
-  } else if (SLICED) {
-    // one slice per workgroup (blockIdx.z), written as linear_splitk_kernel writes it
-    const int n0 = blockIdx.x * G::BN, sl = blockIdx.z;
-    int a, b;
-    split_range(nks, S, sl, a, b);
-    G::template run<BLK>(w, [n0](int r) { return n0 + r; }, xb, K, Mb, K, a, b, sm_lin, acc);
-    float* part = static_cast<float*>(out) + static_cast<size_t>(sl) * M * N;
+    } else {
+      const size_t plane = MODE == kRowsSlice ? static_cast<size_t>(blockIdx.y) * M : 0;
+      float* po = static_cast<float*>(out) + (plane + m0 + m) * N + n0 + 16 * WN * wc + 4 * lg;
 #pragma unroll
-    for (int mt = 0; mt < MTW; ++mt) {
-      const int m = 16 * (MTW * wr + mt) + lr;
-      if (m >= Mb) continue;
-#pragma unroll
-      for (int j = 0; j < WN; ++j)
-        *reinterpret_cast<f32x4*>(part + static_cast<size_t>(m0 + m) * N + n0 + 16 * (WN * wc + j) +
-                                  4 * lg) = acc[j][mt];
-    }
-  } else {
-    const int n0 = blockIdx.x * G::BN;
-    G::template run<BLK>(w, [n0](int r) { return n0 + r; }, xb, K, Mb, K, 0, nks, sm_lin, acc, fold);
-#pragma unroll
-    for (int mt = 0; mt < MTW; ++mt) {
-      const int m = 16 * (MTW * wr + mt) + lr;
-      if (m >= Mb) continue;
-#pragma unroll
-      for (int j = 0; j < WN; ++j)
-        *reinterpret_cast<f32x4*>(static_cast<float*>(out) + static_cast<size_t>(m0 + m) * N + n0 +
-                                  16 * (WN * wc + j) + 4 * lg) = tot[j][mt];
+      for (int j = 0; j < WN; ++j) {
+        if constexpr (TOT) *reinterpret_cast<f32x4*>(po + 16 * j) = tot[j][mt];
+        else *reinterpret_cast<f32x4*>(po + 16 * j) = acc[j][mt];
+      }
     }
   }
 }
@@ -1647,13 +1735,28 @@ static int resident_cus() {
   return cus[dev];
 }
 
-// Slices kve_linear_rows writes: the whole sum (1) when the output tiles alone
-// give the chip a workgroup per CU, else every k-slice (the reductions then sum
-// them, as after kve_linear_splitk). Gate/up always writes its activation.
+// Row tile of a kve_linear_rows launch. Two workgroups share a CU; a round of
+// tiles that leaves at most one per CU takes about 0.62 of a full one, and a
+// tile's fixed cost (first loads, outputs) is that of about 63 rows. Fitted to
+// gate/up, down and o at 200-6154 rows: the tile it picks was within 4 % of the
+// fastest of 128 / 160 / 192 / 256 rows at each.
+static float rows_cost(int rows, int bm, int cols) {
+  const int tiles = cdiv(rows, bm) * cols, slots = 2 * resident_cus();
+  const int rem = tiles % slots;
+  return (tiles / slots + (rem == 0 ? 0.0f : rem <= slots / 2 ? 0.62f : 1.0f)) * (bm + 63);
+}
+
+// Slices kve_linear_rows writes: every k-slice while the partial sums' traffic
+// (written and read back) costs less than one workgroup's walk over all of K,
+// else their sum (1). Gate/up always writes its activation. 3B shapes, slices
+// and their reduction against the sum: down (K 11008) at 1024 rows 61 against
+// 74 us, at 1777 113 against 86; o (K 2048) at 400 rows 17.5 against 18.7, at
+// 700 28 against 20: the lines cross near 157 MB at K 11008 and 52 MB at 2048.
 static int rows_slices(int rows, int N, int K, int mode) {
   if (mode == 2) return 1;
-  const int tiles = (N / RowsCfg::G::BN) * cdiv(rows, RowsCfg::G::XROWS);
-  return tiles >= resident_cus() ? 1 : splitk_slices(N, K);
+  const int S = splitk_slices(N, K);
+  const int64_t traffic = int64_t{8} * S * rows * N;
+  return traffic <= 28000000 + int64_t{11700} * K ? S : 1;
 }
 
 extern "C" int kve_linear_rows_slices(int rows, int out_features, int in_features, int mode) {
@@ -1670,8 +1773,7 @@ extern "C" int kve_linear_rows(const void* x, const void* weight, void* out, int
   KVE_REQUIRE(rows > 0 && mode >= 0 && mode <= 2, "kve_linear_rows: rows %d mode %d", rows, mode);
   KVE_REQUIRE(in_features > 0 && in_features % 64 == 0,
               "kve_linear_rows: in %d (multiple of 64)", in_features);
-  using C = RowsCfg;
-  const int unit = C::G::BN;
+  constexpr int unit = RowsTile<4, 4>::BN;
   KVE_REQUIRE(out_features > 0 && out_features % unit == 0,
               "kve_linear_rows: out %d (multiple of %d)", out_features, unit);
   KVE_REQUIRE(aligned16(x) && aligned16(weight) && aligned16(out),
@@ -1682,28 +1784,41 @@ extern "C" int kve_linear_rows(const void* x, const void* weight, void* out, int
   hipStream_t st = static_cast<hipStream_t>(stream);
   const uint16_t* xp = static_cast<const uint16_t*>(x);
   const uint16_t* wp = static_cast<const uint16_t*>(weight);
-  const int F = out_features / 2;
   const int S = mode == 2 ? 1 : splitk_slices(out_features, in_features);
   const bool sliced = rows_slices(rows, out_features, in_features, mode) > 1;
-  dim3 grid(mode == 2 ? F / (C::G::BN / 2) : out_features / C::G::BN, cdiv(rows, C::G::XROWS),
-            sliced ? S : 1);
-  const size_t lds = C::G::LDS_BYTES;
+  const int N = mode == 2 ? out_features / 2 : out_features;
+  const int nx = out_features / unit, cols = sliced ? nx * S : nx;
+  // 256 rows (no room for the running sum) and 160 or 192, else 128
+  const float c128 = rows_cost(rows, 128, cols), c160 = rows_cost(rows, 160, cols);
+  const float c192 = rows_cost(rows, 192, cols), c256 = rows_cost(rows, 256, cols);
   int rc;
-#define KVE_ROWS(MODE_, SL_, N_)                                                                \
-  do {                                                                                         \
-    static size_t granted_ = 0, granted_b_ = 0;                                                \
-    if (blk)                                                                                   \
-      rc = launch_lds(linear_rows_kernel<MODE_, SL_, C, true>, granted_b_, grid, dim3(C::NT), lds, \
-                      st, xp, wp, out, rows, N_, in_features, S);                              \
-    else                                                                                       \
-      rc = launch_lds(linear_rows_kernel<MODE_, SL_, C>, granted_, grid, dim3(C::NT), lds, st, xp, \
-                      wp, out, rows, N_, in_features, S);                                      \
+#define KVE_ROWS(MODE_, MTW_, NB_)                                                              \
+  do {                                                                                          \
+    using C = RowsTile<MTW_, NB_>;                                                              \
+    static size_t granted_ = 0, granted_b_ = 0;                                                 \
+    const int ny = cdiv(rows, C::BM);                                                           \
+    const dim3 grid(nx* ny, sliced ? S : 1);                                                    \
+    if (blk)                                                                                    \
+      rc = launch_lds(linear_rows_kernel<MODE_, C, true>, granted_b_, grid, dim3(C::NT), C::LDS, st, \
+                      xp, wp, out, rows, N, in_features, S, nx, ny);                            \
+    else                                                                                        \
+      rc = launch_lds(linear_rows_kernel<MODE_, C, false>, granted_, grid, dim3(C::NT), C::LDS, st, \
+                      xp, wp, out, rows, N, in_features, S, nx, ny);                            \
   } while (0)
-  if (mode == 2) KVE_ROWS(2, false, F);
-  else if (mode == 1 && sliced) KVE_ROWS(1, true, out_features);
-  else if (mode == 1) KVE_ROWS(1, false, out_features);
-  else if (sliced) KVE_ROWS(0, true, out_features);
-  else KVE_ROWS(0, false, out_features);
+  if (mode == 2) {
+    if (c256 <= c192 && c256 <= c128) KVE_ROWS(2, 8, 3);
+    else if (c192 <= c128) KVE_ROWS(2, 6, 4);
+    else KVE_ROWS(2, 4, 4);
+  } else if (sliced) {
+    if (c192 <= c128) KVE_ROWS(kRowsSlice, 6, 4);
+    else KVE_ROWS(kRowsSlice, 4, 4);
+  } else if (mode == 1) {
+    if (c160 <= c128) KVE_ROWS(1, 5, 4);
+    else KVE_ROWS(1, 4, 4);
+  } else {
+    if (c160 <= c128) KVE_ROWS(0, 5, 4);
+    else KVE_ROWS(0, 4, 4);
+  }
 #undef KVE_ROWS
   if (rc) return rc;
   return check_launch("kve_linear_rows");

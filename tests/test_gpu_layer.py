@@ -865,3 +865,32 @@ def test_blocked_linear_rows_equals_row_major(gpu_lib, M, N, K, mode):
     if mode == kernels.ROWS_GATE_UP:
         got = kernels.from_blocked(got, M)
     assert torch.equal(got, want)
+
+
+# (M, N, mode): the row tile each launch takes (128, 160, 192 or 256 rows) with a
+# row less or more than whole tiles; K 11008 has 43 k-steps per slice, K 192 six in all
+@pytest.mark.parametrize("M,N,K,mode", [
+    (1023, 22016, 192, 2), (1025, 22016, 192, 2), (2881, 22016, 192, 2), (127, 9728, 896, 2),
+    (4639, 2560, 2048, 1), (4641, 2048, 2048, 0), (1791, 2048, 11008, 0), (1793, 2048, 1984, 0),
+    (383, 2048, 11008, 0), (385, 2048, 11008, 0), (257, 2048, 2752, 0), (193, 1152, 896, 1)])
+@pytest.mark.parametrize("blocked", [True, False])
+def test_linear_rows_tile_edges(gpu_lib, M, N, K, mode, blocked):
+    """Rows just short of and just past a row tile, odd k-steps per slice, in
+    both layouts: bit for bit the split-K kernels' rows."""
+    g = torch.Generator().manual_seed(M + N + K + mode)
+    x = torch.randn(M, K, generator=g).bfloat16().to(DEV)
+    W = (0.03 * torch.randn(N, K, generator=g)).bfloat16().to(DEV)
+    want = _splitk_rows_reference(x, W, mode)
+    if blocked:
+        got = kernels.linear_rows(kernels.to_blocked(x), kernels.to_blocked(W), mode, blocked=True,
+                                  rows=M)
+        if mode == kernels.ROWS_GATE_UP:
+            got = kernels.from_blocked(got, M)
+    else:
+        got = kernels.linear_rows(x, W, mode)
+    if mode != kernels.ROWS_GATE_UP:
+        t = got[0].clone() if mode == kernels.ROWS_RESIDUAL else torch.zeros_like(got[0]) + got[0]
+        for s in range(1, got.shape[0]):
+            t += got[s]
+        got = t
+    assert torch.equal(got, want)
