@@ -410,6 +410,28 @@ int kve_qkv_part_rope(const float* partials, int slices, const void* bias, const
                       int block_size, void* stream);
 
 /*
+ * kve_qkv_part_rope_to: kve_qkv_part_rope with row m's rotated q written to row
+ * q_rows[m] (int64) of q_out [q_capacity, Hq, head_dim] instead of row m (q_rows
+ * NULL: row m), so that a packed prefill's q lands in the padded [seq, token]
+ * rows its attention reads. A row index outside [0, q_capacity) drops that q.
+ */
+int kve_qkv_part_rope_to(const float* partials, int slices, const void* bias, const void* cos,
+                         const void* sin, const int32_t* slots, const int64_t* q_rows,
+                         int q_capacity, void* q_out, void* k_pool, void* v_pool, int rows,
+                         int num_q_heads, int num_kv_heads, int head_dim, int block_size,
+                         void* stream);
+
+/*
+ * kve_gather_rows: dst row j = src row index[j], j < rows, for bf16 rows of
+ * `cols` (a multiple of 32) values: src [src_rows, cols] row-major, dst
+ * row-major or blocked (layout), index int64. An index outside [0, src_rows)
+ * leaves its row of dst as it is. No counterpart in the reference, whose
+ * prefill takes one sequence at a time.
+ */
+int kve_gather_rows(const void* src, const int64_t* index, void* dst, int rows, int src_rows,
+                    int cols, int layout, void* stream);
+
+/*
  * kve_gate_up_silu: act = cast(silu(xn Wg^T)) * (xn Wu^T) for normalised rows
  * xn [rows <= 160, hidden] and the [gate|up] weight [2*ffn, hidden] (Qwen2MLP
  * up to down_proj, modeling_qwen2.py:35-48). A row's result does not depend

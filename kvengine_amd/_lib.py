@@ -40,6 +40,8 @@ EXPORTS = (
     "kve_kv_slots",
     "kve_qkv_rope",
     "kve_qkv_part_rope",
+    "kve_qkv_part_rope_to",
+    "kve_gather_rows",
     "kve_gate_up_silu",
     "kve_linear_rows",
     "kve_linear_rows_slices",
@@ -85,6 +87,8 @@ _SIGS = {
     "kve_kv_slots": (I, [P, P, P, P, I, I, I, I, I, I, P, P]),
     "kve_qkv_rope": (I, [P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P]),
     "kve_qkv_part_rope": (I, [P, I, P, P, P, P, P, P, P, I, I, I, I, I, P]),
+    "kve_qkv_part_rope_to": (I, [P, I, P, P, P, P, P, I, P, P, P, I, I, I, I, I, P]),
+    "kve_gather_rows": (I, [P, P, P, I, I, I, I, P]),
     "kve_gate_up_silu": (I, [P, P, P, I, I, I, I, P]),
     "kve_linear_rows": (I, [P, P, P, I, I, I, I, I, P]),
     "kve_linear_rows_slices": (I, [I, I, I, I]),

@@ -641,8 +641,11 @@ __global__ __launch_bounds__(C::NT) void linear_splitk_kernel(const uint16_t* x,
 // projection's bf16 output added to the bf16 residual), then xn =
 // w * cast(r * rsqrt(mean(r^2) + eps)) as Qwen2RMSNorm. Thread t owns the
 // 4-column groups t, t + 256 (H <= 2048), so each load instruction reads
-// contiguous memory; the slices' loads go out eight at a time and are summed
-// in order 0, 1, ..., S-1.
+// contiguous memory; the slices' loads go out SB at a time and are summed in
+// order 0, 1, ..., S-1. SB = 8, or 1 for whole sums (S = 1, a prefill's
+// projections): with eight loads of the one slice a row of 2048 columns read
+// 64 KB from L1 for its 8 KB (3B at 6154 rows 35 -> 24 us).
+template <int SB>
 __global__ __launch_bounds__(256) void residual_norm_kernel(const float* part, int S,
                                                             uint16_t* residual,
                                                             const uint16_t* norm_w, float eps,
@@ -663,10 +666,10 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(const float* part, i
     rv[j] = reinterpret_cast<const u32x2*>(rrow)[g[j]];
     wvv[j] = reinterpret_cast<const u32x2*>(norm_w)[g[j]];
   }
-  for (int s0 = 0; s0 < S; s0 += 8) {
-    f32x4 t[8][NG];
+  for (int s0 = 0; s0 < S; s0 += SB) {
+    f32x4 t[SB][NG];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < SB; ++i) {
       const f32x4* ps =
           reinterpret_cast<const f32x4*>(part + (static_cast<size_t>(min(s0 + i, S - 1)) * M + m) * H);
 #pragma unroll
@@ -676,7 +679,7 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(const float* part, i
     // by a select): with a branch here the compiler sank each slice's loads
     // into it and waited for them one slice at a time.
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < SB; ++i) {
       const bool first = s0 + i == 0, live = s0 + i < S;
 #pragma unroll
       for (int j = 0; j < NG; ++j) {
@@ -858,6 +861,33 @@ __global__ __launch_bounds__(128) void qkv_rope_kernel(QkvRopeArgs a) {
   }
 }
 
+// dst row j = src row index[j] (bf16 [src_rows, C] -> [rows, C], row-major or
+// blocked; an index outside src leaves its row as it is): a packed prefill's
+// attention rows for o_proj. One workgroup per 16 rows, one wave per row, four
+// 16-byte units per lane in flight, so a workgroup writes whole blocked 1 KB
+// pieces at about the same time. The index_select it replaces gave row-major
+// rows; o_proj takes 59 us on blocked rows and 73 on row-major ones (3B, 6154).
+__global__ __launch_bounds__(1024) void gather_rows_kernel(const uint16_t* src, const int64_t* index,
+                                                           uint16_t* dst, int rows, int src_rows,
+                                                           int C, int blocked) {
+  constexpr int NU = 4;
+  const int j = blockIdx.x * 16 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (j >= rows) return;
+  const int64_t r = index[j];
+  if (r < 0 || r >= src_rows) return;
+  const u32x4* s = reinterpret_cast<const u32x4*>(src + static_cast<size_t>(r) * C);
+  const int nu = C / 8;
+  for (int u0 = l; u0 < nu; u0 += 64 * NU) {
+    u32x4 v[NU];
+#pragma unroll
+    for (int i = 0; i < NU; ++i) v[i] = s[min(u0 + 64 * i, nu - 1)];
+#pragma unroll
+    for (int i = 0; i < NU; ++i)
+      if (u0 + 64 * i < nu)
+        *reinterpret_cast<u32x4*>(dst + mat_off(j, 8 * (u0 + 64 * i), C, C, blocked)) = v[i];
+  }
+}
+
 struct QkvPartArgs {
   const float* part;     // [S, M, (Hq + 2 Hkv) D] k-slice partial products
   const uint16_t* bias;  // [(Hq + 2 Hkv) D]
@@ -867,7 +897,8 @@ struct QkvPartArgs {
   uint16_t* q_out;       // [M, Hq, D]
   uint16_t* k_pool;      // [NB, Hkv, bs, D]
   uint16_t* v_pool;      // [NB, Hkv, D, bs]
-  int S, M, Hq, Hkv, bs;
+  const int64_t* q_rows; // [M] row of q_out each row's q goes to (null: its own)
+  int S, M, Hq, Hkv, bs, q_cap;
 };
 
 // Epilogue of the split-K [q|k|v] projection: per row, each column's slices
@@ -878,12 +909,14 @@ struct QkvPartArgs {
 // dealt 256 to a workgroup, so every thread makes one round trip for its
 // partials (the 3B's 320 groups on one workgroup took two: 3B verify pass at
 // 5 / 40 / 160 rows 2414 / 2735 / 3640 -> 2349 / 2677 / 3602 us).
-template <int D>
+// SB: slices loaded per batch, 8, or 1 for whole sums (S = 1; 3B at 6154 rows
+// 37 -> 26 us, as in residual_norm_kernel).
+template <int D, int SB>
 __global__ __launch_bounds__(256) void qkv_part_rope_kernel(QkvPartArgs a) {
   constexpr int half = D / 2;
   constexpr int GPH = half / 4;  // 4-column groups per head half
-  constexpr int SB = 8;          // slices loaded per batch
   const int m = blockIdx.x;
+  const int64_t qm = a.q_rows ? a.q_rows[m] : m;
   const int N = (a.Hq + 2 * a.Hkv) * D;
   const int slot = a.slots[m];
   const int blk = slot >= 0 ? slot / a.bs : 0, off = slot >= 0 ? slot - blk * a.bs : 0;
@@ -932,7 +965,8 @@ __global__ __launch_bounds__(256) void qkv_part_rope_kernel(QkvPartArgs a) {
     if (rot) {
       uint16_t* dst;
       if (h < a.Hq) {
-        dst = a.q_out + (static_cast<size_t>(m) * a.Hq + h) * D;
+        if (qm < 0 || qm >= a.q_cap) continue;  // a row index outside q_out is dropped
+        dst = a.q_out + (static_cast<size_t>(qm) * a.Hq + h) * D;
       } else {
         if (slot < 0) continue;
         dst = a.k_pool + ((static_cast<size_t>(blk) * a.Hkv + (h - a.Hq)) * a.bs + off) * D;
@@ -1541,7 +1575,8 @@ extern "C" int kve_residual_norm(const float* partials, int slices, void* residu
               "kve_residual_norm: buffers must be 16-byte aligned");
   KVE_REQUIRE(layout == KVE_LAYOUT_ROWS || (layout == KVE_LAYOUT_BLOCKED && hidden % 32 == 0),
               "kve_residual_norm: layout %d with hidden %d", layout, hidden);
-  hipLaunchKernelGGL(residual_norm_kernel, dim3(rows), dim3(256), 0, static_cast<hipStream_t>(stream),
+  const auto kernel = slices == 1 ? residual_norm_kernel<1> : residual_norm_kernel<8>;
+  hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, static_cast<hipStream_t>(stream),
                      partials, slices, static_cast<uint16_t*>(residual),
                      static_cast<const uint16_t*>(norm_weight), eps, static_cast<uint16_t*>(xn), rows,
                      hidden, layout == KVE_LAYOUT_BLOCKED ? 1 : 0);
@@ -1626,11 +1661,11 @@ extern "C" int kve_qkv_rope(const void* xn, const void* weight, const void* bias
   return check_launch("kve_qkv_rope");
 }
 
-extern "C" int kve_qkv_part_rope(const float* partials, int slices, const void* bias,
-                                 const void* cos, const void* sin, const int32_t* slots,
-                                 void* q_out, void* k_pool, void* v_pool, int rows,
-                                 int num_q_heads, int num_kv_heads, int head_dim, int block_size,
-                                 void* stream) {
+extern "C" int kve_qkv_part_rope_to(const float* partials, int slices, const void* bias,
+                                    const void* cos, const void* sin, const int32_t* slots,
+                                    const int64_t* q_rows, int q_capacity, void* q_out,
+                                    void* k_pool, void* v_pool, int rows, int num_q_heads,
+                                    int num_kv_heads, int head_dim, int block_size, void* stream) {
   clear_error();
   if (rows == 0) return KVE_OK;
   KVE_REQUIRE(partials && bias && cos && sin && slots && q_out && k_pool && v_pool,
@@ -1652,6 +1687,8 @@ extern "C" int kve_qkv_part_rope(const float* partials, int slices, const void* 
   a.q_out = static_cast<uint16_t*>(q_out);
   a.k_pool = static_cast<uint16_t*>(k_pool);
   a.v_pool = static_cast<uint16_t*>(v_pool);
+  a.q_rows = q_rows;
+  a.q_cap = q_rows ? q_capacity : rows;
   a.S = slices;
   a.M = rows;
   a.Hq = num_q_heads;
@@ -1659,10 +1696,40 @@ extern "C" int kve_qkv_part_rope(const float* partials, int slices, const void* 
   a.bs = block_size;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid(rows, cdiv((num_q_heads + 2 * num_kv_heads) * (head_dim / 8), 256));
-  if (head_dim == 64) hipLaunchKernelGGL(qkv_part_rope_kernel<64>, grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(qkv_part_rope_kernel<128>, grid, dim3(256), 0, st, a);
+  const auto kernel = head_dim == 64
+                          ? (slices == 1 ? qkv_part_rope_kernel<64, 1> : qkv_part_rope_kernel<64, 8>)
+                          : (slices == 1 ? qkv_part_rope_kernel<128, 1> : qkv_part_rope_kernel<128, 8>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, a);
   return check_launch("kve_qkv_part_rope");
 }
+
+extern "C" int kve_qkv_part_rope(const float* partials, int slices, const void* bias,
+                                 const void* cos, const void* sin, const int32_t* slots,
+                                 void* q_out, void* k_pool, void* v_pool, int rows,
+                                 int num_q_heads, int num_kv_heads, int head_dim, int block_size,
+                                 void* stream) {
+  return kve_qkv_part_rope_to(partials, slices, bias, cos, sin, slots, nullptr, 0, q_out, k_pool,
+                              v_pool, rows, num_q_heads, num_kv_heads, head_dim, block_size, stream);
+}
+
+extern "C" int kve_gather_rows(const void* src, const int64_t* index, void* dst, int rows,
+                               int src_rows, int cols, int layout, void* stream) {
+  clear_error();
+  if (rows == 0) return KVE_OK;
+  KVE_REQUIRE(src && index && dst, "kve_gather_rows: null pointer argument");
+  KVE_REQUIRE(rows > 0 && src_rows > 0 && cols > 0 && cols % 32 == 0,
+              "kve_gather_rows: %d of %d rows of %d (a multiple of 32)", rows, src_rows, cols);
+  KVE_REQUIRE(aligned16(src) && aligned16(dst) && (reinterpret_cast<uintptr_t>(index) & 7) == 0,
+              "kve_gather_rows: src and dst must be 16-byte aligned, index 8-byte");
+  KVE_REQUIRE(layout == KVE_LAYOUT_ROWS || layout == KVE_LAYOUT_BLOCKED, "kve_gather_rows: layout %d",
+              layout);
+  hipLaunchKernelGGL(gather_rows_kernel, dim3(cdiv(rows, 16)), dim3(1024), 0,
+                     static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(src), index,
+                     static_cast<uint16_t*>(dst), rows, src_rows, cols,
+                     layout == KVE_LAYOUT_BLOCKED ? 1 : 0);
+  return check_launch("kve_gather_rows");
+}
+
 
 extern "C" int kve_gate_up_silu(const void* xn, const void* weight, void* act, int rows, int hidden,
                                 int ffn, int layout, void* stream) {

@@ -451,6 +451,7 @@ def forward_packed_wide(model, ids: torch.Tensor, dst: torch.Tensor, B: int, T: 
     inner = model.model
     layers = inner.layers
     N = ids.numel()
+    dst = dst.contiguous()
     residual = inner.embed_tokens(ids).contiguous()
     start = kv.lens.index_select(0, rows).to(torch.long)
     positions = start[:, None] + torch.arange(T, device=ids.device)[None, :]
@@ -461,11 +462,11 @@ def forward_packed_wide(model, ids: torch.Tensor, dst: torch.Tensor, B: int, T: 
     slots = kernels.kv_slots(kv.tables, kv.lens, B, T, kv.block_size, kv.k.shape[1], seq_rows=rows,
                              q_lens=q_lens).index_select(0, dst)
     Hq = _q_heads(model, kv)
-    # padded rows are never read (q_lens masks them); zero them once anyway
-    q_pad = torch.zeros(B * T, Hq * D, dtype=residual.dtype, device=ids.device)
-    # blocked weights: the normalised rows and the gate/up activations between the
-    # launches are blocked matrices (o_proj reads the gathered attention rows
-    # row-major); the final hidden states are row-major
+    # rows past a sequence's q_len are never read (q_lens masks them)
+    q_pad = torch.empty(B * T, Hq * D, dtype=residual.dtype, device=ids.device)
+    # blocked weights: the normalised rows, the gathered attention rows and the
+    # gate/up activations between the launches are blocked matrices; the final
+    # hidden states are row-major
     blk = _has_blocked(model)
     first = layers[0].input_layernorm
     xn = kernels.rmsnorm(residual, first.weight, first.variance_epsilon, blocked=blk)
@@ -478,11 +479,12 @@ def forward_packed_wide(model, ids: torch.Tensor, dst: torch.Tensor, B: int, T: 
         mlp = layer.mlp
         part = _wide_proj(xn, attn.qkv_weight_blk if blk else attn.qkv_weight, kernels.ROWS_QKV,
                           blocked=blk, rows=N)
-        q = kernels.qkv_part_rope(part, attn.qkv_bias, cos, sin, slots, kv.k[li], kv.v[li], Hq, N)
-        q_pad.index_copy_(0, dst, q.view(N, Hq * D))
+        kernels.qkv_part_rope(part, attn.qkv_bias, cos, sin, slots, kv.k[li], kv.v[li], Hq, N,
+                              q_out=q_pad, q_rows=dst)
         out = layer_attn(q_pad.view(B, T, Hq, D), li, attn.scaling)
-        o_in = out.reshape(B * T, Hq * D).index_select(0, dst)
-        part = _wide_proj(o_in, attn.o_proj.weight, kernels.ROWS_RESIDUAL)
+        o_in = kernels.gather_rows(out.view(B * T, Hq * D), dst, blocked=blk)
+        part = _wide_proj(o_in, attn.o_weight_blk if blk else attn.o_proj.weight,
+                          kernels.ROWS_RESIDUAL, blocked=blk, rows=N)
         post = layer.post_attention_layernorm
         xn = kernels.residual_norm(part, part.shape[0], residual, post.weight, post.variance_epsilon,
                                    xn=xn, blocked=blk)

@@ -656,9 +656,11 @@ def qkv_rope(xn: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, cos: to
 
 def qkv_part_rope(partials: torch.Tensor, bias: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                   slots: torch.Tensor, k_layer: torch.Tensor, v_layer: torch.Tensor,
-                  num_q_heads: int, rows: int, q_out: torch.Tensor | None = None) -> torch.Tensor:
+                  num_q_heads: int, rows: int, q_out: torch.Tensor | None = None,
+                  q_rows: torch.Tensor | None = None) -> torch.Tensor:
     """Split-K [q|k|v] partials [S, rows, (Hq + 2 Hkv) D] -> sum + bias -> RoPE; k/v
-    written at `slots`, rotated q [rows, Hq, D] returned (as qkv_rope)."""
+    written at `slots`, rotated q [rows, Hq, D] returned (as qkv_rope). q_rows
+    (int64 [rows]): row m's q goes to row q_rows[m] of q_out [any, Hq, D]."""
     dev = partials.device
     NB, Hkv, bs, D = k_layer.shape
     N = (num_q_heads + 2 * Hkv) * D
@@ -671,13 +673,39 @@ def qkv_part_rope(partials: torch.Tensor, bias: torch.Tensor, cos: torch.Tensor,
     _check_i32(slots, "slots", dev)
     _need(slots.numel() >= rows, "one slot per row")
     if q_out is None:
+        _need(q_rows is None, "q_rows needs q_out")
         q_out = torch.empty(rows, num_q_heads, D, dtype=torch.bfloat16, device=dev)
-    rc = _lib.lib().kve_qkv_part_rope(partials.data_ptr(), partials.shape[0], bias.data_ptr(),
-                                      cos.data_ptr(), sin.data_ptr(), slots.data_ptr(),
-                                      q_out.data_ptr(), k_layer.data_ptr(), v_layer.data_ptr(), rows,
-                                      num_q_heads, Hkv, D, bs, _stream(dev))
+    cap = q_out.numel() // (num_q_heads * D)
+    if q_rows is not None:
+        _check_index(q_rows, rows, dev)
+        _need(q_out.dtype == torch.bfloat16 and q_out.is_contiguous()
+              and q_out.numel() == cap * num_q_heads * D, "q_out [any, Hq, D]")
+    rc = _lib.lib().kve_qkv_part_rope_to(partials.data_ptr(), partials.shape[0], bias.data_ptr(),
+                                         cos.data_ptr(), sin.data_ptr(), slots.data_ptr(),
+                                         _ptr(q_rows), cap, q_out.data_ptr(), k_layer.data_ptr(),
+                                         v_layer.data_ptr(), rows, num_q_heads, Hkv, D, bs,
+                                         _stream(dev))
     _lib.check(rc, "kve_qkv_part_rope")
     return q_out
+
+
+def _check_index(index: torch.Tensor, rows: int, dev) -> None:
+    _need(index.dtype == torch.int64 and index.device == dev and index.is_contiguous()
+          and index.numel() == rows, "row indices must be contiguous int64, one per row")
+
+
+def gather_rows(src: torch.Tensor, index: torch.Tensor, blocked: bool = False) -> torch.Tensor:
+    """Rows index[j] of the bf16 matrix src [R, C] (int64 index), row-major [N, C]
+    or as a blocked matrix."""
+    _need(src.dim() == 2 and src.dtype == torch.bfloat16 and src.is_contiguous(), "src [R, C] bf16")
+    n, C = index.numel(), src.shape[1]
+    _check_index(index, n, src.device)
+    dst = (blocked_matrix(n, C, src.device) if blocked
+           else torch.empty(n, C, dtype=src.dtype, device=src.device))
+    rc = _lib.lib().kve_gather_rows(src.data_ptr(), index.data_ptr(), dst.data_ptr(), n,
+                                    src.shape[0], C, _layout(blocked), _stream(src.device))
+    _lib.check(rc, "kve_gather_rows")
+    return dst
 
 
 def gate_up_silu(xn: torch.Tensor, weight: torch.Tensor, act: torch.Tensor | None = None,

@@ -894,3 +894,32 @@ def test_linear_rows_tile_edges(gpu_lib, M, N, K, mode, blocked):
             t += got[s]
         got = t
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("n,R,C", [(1, 1, 32), (17, 40, 896), (160, 333, 2048), (33, 33, 96)])
+def test_gather_rows_and_scattered_q(gpu_lib, n, R, C):
+    """kve_gather_rows copies the indexed rows in either layout (an index outside
+    src leaves its row as it is); kve_qkv_part_rope_to with a row map writes the
+    q of kve_qkv_part_rope to the mapped rows and touches no other."""
+    g = torch.Generator().manual_seed(n + R + C)
+    src = torch.randn(R, C, generator=g).bfloat16().to(DEV)
+    idx = torch.randperm(R, generator=g)[:n].to(DEV) if n <= R else torch.zeros(n, dtype=torch.long)
+    assert torch.equal(kernels.gather_rows(src, idx), src[idx])
+    assert torch.equal(kernels.from_blocked(kernels.gather_rows(src, idx, blocked=True), n), src[idx])
+    Hq, Hkv, D, bs, S = 4, 2, 64, 16, (1 if n % 2 else 3)
+    N = (Hq + 2 * Hkv) * D
+    part = torch.randn(S, n, N, generator=g).to(DEV)
+    bias = torch.randn(N, generator=g).bfloat16().to(DEV)
+    cos, sin = (torch.randn(n, D, generator=g).bfloat16().to(DEV) for _ in range(2))
+    slots = torch.arange(n, dtype=torch.int32, device=DEV)
+    pools = [[torch.zeros(-(-n // bs), Hkv, *s, dtype=torch.bfloat16, device=DEV)
+              for s in ((bs, D), (D, bs))] for _ in range(2)]
+    want = kernels.qkv_part_rope(part, bias, cos, sin, slots, *pools[0], Hq, n)
+    out = torch.full((R + 3, Hq * D), 7.0, dtype=torch.bfloat16, device=DEV)
+    kernels.qkv_part_rope(part, bias, cos, sin, slots, *pools[1], Hq, n, q_out=out, q_rows=idx)
+    assert torch.equal(out[idx], want.view(n, Hq * D))
+    rest = torch.ones(R + 3, dtype=torch.bool, device=DEV)
+    rest[idx] = False
+    assert (out[rest] == 7.0).all()
+    for a, b in zip(*pools):
+        assert torch.equal(a, b)
