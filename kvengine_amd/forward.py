@@ -222,7 +222,7 @@ def forward_hidden(model, input_ids: torch.Tensor, kv: DeviceKV, rows: torch.Ten
                 return _forward_splitk(model, input_ids, kv, rows, max_ctx, q_lens, attn_order,
                                        blocked_out=blocked_out)
             return _forward_small(model, input_ids, kv, rows, max_ctx, q_lens, attn_order)
-        if n <= SPLITK_MAX_ROWS and _wide_ok(model, n):
+        if _wide_ok(model, n):
             return _forward_splitk(model, input_ids, kv, rows, max_ctx, q_lens, attn_order, wide=True,
                                    blocked_out=blocked_out)
         return _forward_fused(model, input_ids, kv, rows, max_ctx, q_lens, attn_order)
@@ -381,7 +381,10 @@ def forward_packed(model, ids: torch.Tensor, dst: torch.Tensor, B: int, T: int, 
     projections run on the N real rows only; RoPE + KV write and attention run
     on the padded [B, T] layout, which packed rows are scattered into and
     gathered back from. Same per-sequence semantics as forward_hidden over the
-    padded [B, T] batch; the caller commits lengths afterwards."""
+    padded [B, T] batch; the caller commits lengths afterwards. Models whose
+    shapes fit (_wide_ok) take forward_packed_wide."""
+    if _wide_ok(model, ids.numel()):
+        return forward_packed_wide(model, ids, dst, B, T, kv, rows, max_ctx, q_lens, attn_order)
     inner = model.model
     layers = inner.layers
     a0 = layers[0].self_attn
@@ -575,10 +578,10 @@ def _forward_splitk(model, input_ids, kv: DeviceKV, rows, max_ctx, q_lens, attn_
     the RMSNorm in its prologue + SiLU*up, down_proj k-slices, residual add +
     the next layer's RMSNorm (the final norm after the last layer). The KV
     slots of the new tokens are resolved once.
-    wide (up to 160 rows): o_proj runs as k-slices + residual add + RMSNorm and
+    wide (any number of rows): o_proj runs as k-slices + residual add + RMSNorm and
     gate/up on the normalised rows, and the QKV projection as k-slices too, with
     its bias / RoPE / KV write in a separate epilogue launch (eight per layer):
-    these are the sums kve_linear_rows reproduces for a prefill.
+    above SPLITK_MAX_ROWS the same sums come from kve_linear_rows.
     With blocked weights the normalised rows, the attention output (wide) and
     the gate/up activations between the launches are blocked matrices; the
     final hidden states are row-major [B, T, H] unless blocked_out."""
@@ -586,7 +589,7 @@ def _forward_splitk(model, input_ids, kv: DeviceKV, rows, max_ctx, q_lens, attn_
     layers = inner.layers
     B, T = input_ids.shape
     n = B * T
-    blk = _has_blocked(model) and n <= SPLITK_MAX_ROWS
+    blk = _has_blocked(model)
     fused_o = not wide and SPLITK_FUSED_O and n <= SPLITK_FUSED_O_ROWS
     residual, cos, sin = _prologue(model, input_ids, kv, rows, max_ctx)
     slots = kernels.kv_slots(kv.tables, kv.lens, B, T, kv.block_size, kv.k.shape[1], seq_rows=rows,
@@ -604,7 +607,7 @@ def _forward_splitk(model, input_ids, kv: DeviceKV, rows, max_ctx, q_lens, attn_
         mlp = layer.mlp
         if blk:
             if wide:
-                part = kernels.linear_splitk(xn, attn.qkv_weight_blk, blocked=True, rows=n)
+                part = _wide_proj(xn, attn.qkv_weight_blk, kernels.ROWS_QKV, blocked=True, rows=n)
                 q = kernels.qkv_part_rope(part, attn.qkv_bias, cos, sin, slots, kv.k[li], kv.v[li],
                                           Hq, n).view(B, T, Hq, -1)
             else:
@@ -615,7 +618,8 @@ def _forward_splitk(model, input_ids, kv: DeviceKV, rows, max_ctx, q_lens, attn_
                 kernels.linear_residual(out.view(n, -1), attn.o_weight_blk, residual, blocked_w=True)
             else:
                 out = layer_attn(q, li, attn.scaling, blocked=True)
-                part = kernels.linear_splitk(out, attn.o_weight_blk, blocked=True, rows=n)
+                part = _wide_proj(out, attn.o_weight_blk, kernels.ROWS_RESIDUAL, blocked=True,
+                                  rows=n)
         else:
             if wide:
                 part = _wide_proj(xn, attn.qkv_weight, kernels.ROWS_QKV)
@@ -639,8 +643,9 @@ def _forward_splitk(model, input_ids, kv: DeviceKV, rows, max_ctx, q_lens, attn_
                                        post.variance_epsilon, xn=xn, blocked=blk)
         if blk:
             if not fused_o:
-                act = kernels.gate_up_silu(xn, mlp.gate_up_weight_blk, blocked=True, rows=n)
-            part = kernels.linear_splitk(act, mlp.down_weight_blk, blocked=True, rows=n)
+                act = _wide_proj(xn, mlp.gate_up_weight_blk, kernels.ROWS_GATE_UP, blocked=True,
+                                 rows=n)
+            part = _wide_proj(act, mlp.down_weight_blk, kernels.ROWS_RESIDUAL, blocked=True, rows=n)
         else:
             if not fused_o:
                 act = _wide_proj(xn, mlp.gate_up_weight, kernels.ROWS_GATE_UP)
