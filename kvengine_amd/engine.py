@@ -45,6 +45,7 @@ from dataclasses import dataclass, field
 import torch
 
 from . import kernels
+from .capture import no_gc
 from .forward import (SPLITK_MAX_ROWS, _fusable, forward_hidden, forward_packed,
                       forward_packed_wide, invariant_gemm_rows, blocked_forward)
 from .model import lm_head_blocked
@@ -385,7 +386,7 @@ class SpecEngine:
             torch.cuda.current_stream().wait_stream(s)
             g = torch.cuda.CUDAGraph()
             self._snapshot_state()
-            with torch.cuda.graph(g):
+            with no_gc(), torch.cuda.graph(g):
                 self._device_iteration(b, ctx)
             self._restore_state()
             b.graphs[ctx] = g
@@ -565,7 +566,7 @@ class SpecEngine:
             if cap is None:
                 cap = self._cap_streams[id(model)] = torch.cuda.Stream(device=self.device)
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g, stream=cap):
+            with no_gc(), torch.cuda.graph(g, stream=cap):
                 run()
             ent.graph = g
         else:

@@ -37,6 +37,7 @@ it passes 896 tokens), so a replayed iteration gives the eager iteration's bits.
 
 from __future__ import annotations
 
+import gc
 import time
 import weakref
 from dataclasses import dataclass, field
@@ -44,6 +45,7 @@ from dataclasses import dataclass, field
 import torch
 
 from . import kernels
+from .capture import no_gc
 from .decode import AUTO_EOS, _resolve_eos, _sync, argmax_rows
 from .forward import forward_hidden
 from .model import lm_head_weight
@@ -143,6 +145,9 @@ class _IterationGraphs:
                tuple(t.data_ptr() for p in (tp, dp) for t in (p.tables, p.lens, p.k, p.v)))
         g = _GRAPHS.get(key)
         if g is None:
+            # dead models' and pools' graphs (kept by reference cycles until a
+            # collection) go now, not while this entry's iterations are captured
+            gc.collect()
             g = _GRAPHS[key] = _IterationGraphs(t_cache.pool, k)
             for obj in (target, draft, t_cache.pool, d_cache.pool):
                 weakref.finalize(obj, _GRAPHS.pop, key, None)
@@ -237,7 +242,7 @@ class _IterationGraphs:
             with torch.cuda.stream(s):
                 self._iteration(u, ctx)
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g, stream=s):
+            with no_gc(), torch.cuda.graph(g, stream=s):
                 self._iteration(u, ctx)
             cur.wait_stream(s)
             self.graphs[(u, ctx)] = g
