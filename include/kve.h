@@ -464,6 +464,31 @@ int kve_linear_rows(const void* x, const void* weight, void* out, int rows, int 
 /* Slices kve_linear_rows writes for these sizes on the current device (0: bad sizes). */
 int kve_linear_rows_slices(int rows, int out_features, int in_features, int mode);
 
+/*
+ * kve_small_pass: every layer of a decode pass of at most 64 rows in one host
+ * call (the layer loop of forward.py:187-208): per layer kve_fused_qkv,
+ * kve_paged_verify_attn, kve_linear_residual (o_proj), kve_fused_gate_up and
+ * kve_linear_residual (down_proj), then kve_rmsnorm of the residual into `out`.
+ * layer_ptrs: host array of 9 device pointers per layer: input norm weight,
+ *      [q|k|v] weight, its bias, K pool, V pool, o_proj weight, post-attention
+ *      norm weight, [gate|up] weight, down_proj weight (weights in `layout`).
+ * layer_consts: host array of 3 floats per layer: input norm eps,
+ *      post-attention norm eps, softmax scale.
+ * residual [rows, hidden] bf16 is updated in place; q and attn_out [2, rows,
+ * num_q_heads * head_dim] and act [2, rows, ffn] are scratch that the layers
+ * rewrite in turn; the other arguments are those of the calls it makes. Both
+ * arrays are read before it returns.
+ */
+int kve_small_pass(const void* const* layer_ptrs, const float* layer_consts, int num_layers,
+                   void* residual, const void* cos, const void* sin, void* q, void* attn_out,
+                   void* act, const int32_t* block_tables, const int32_t* seq_rows,
+                   const int32_t* start_pos, const int32_t* q_lens, int num_seqs, int q_len,
+                   int hidden, int ffn, int num_q_heads, int num_kv_heads, int head_dim,
+                   int block_size, int max_blocks, int num_rows, int num_blocks, int max_ctx,
+                   int unit_blocks, int key_waves, const void* plan, void* workspace,
+                   size_t workspace_bytes, const void* norm_weight, float norm_eps, void* out,
+                   int layout, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

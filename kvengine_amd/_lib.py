@@ -45,6 +45,7 @@ EXPORTS = (
     "kve_gate_up_silu",
     "kve_linear_rows",
     "kve_linear_rows_slices",
+    "kve_small_pass",
 )
 
 DTYPE_F32 = 0
@@ -92,6 +93,8 @@ _SIGS = {
     "kve_gate_up_silu": (I, [P, P, P, I, I, I, I, P]),
     "kve_linear_rows": (I, [P, P, P, I, I, I, I, I, P]),
     "kve_linear_rows_slices": (I, [I, I, I, I]),
+    "kve_small_pass": (I, [P, P, I, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, I, I, I,
+                           I, I, P, P, SZ, P, F, P, I, P]),
 }
 
 

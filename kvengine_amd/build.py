@@ -19,7 +19,7 @@ BUILD_DIR = os.path.join(HERE, "_build")
 ARCH = "gfx950"
 
 SOURCES = ["kve_runtime.hip", "kve_attn.hip", "kve_kvcache.hip", "kve_lmhead.hip",
-           "kve_layer.hip", "kve_linear.hip"]
+           "kve_layer.hip", "kve_linear.hip", "kve_pass.hip"]
 
 # Per-file flags: the fused layer and projection kernels must round every
 # product and sum like the torch ops they replace, so no multiply-add

@@ -514,35 +514,29 @@ def _prologue(model, input_ids, kv: DeviceKV, rows, max_ctx):
 def _forward_small(model, input_ids, kv: DeviceKV, rows, max_ctx, q_lens, attn_order):
     """Five launches per layer: fused QKV (RMSNorm, bias, RoPE, KV write),
     attention (+ its split merge), o_proj + residual, fused gate/up (RMSNorm,
-    SiLU*up), down_proj + residual. The residual stream is updated in place."""
+    SiLU*up), down_proj + residual, all issued by one host call. The residual
+    stream is updated in place."""
     inner = model.model
     B, T = input_ids.shape
     blk = _has_blocked(model)  # weights only: the kernels' other operands stay row-major
     residual, cos, sin = _prologue(model, input_ids, kv, rows, max_ctx)
-    layer_attn = LayerAttention(kv, rows, B, T, _q_heads(model, kv), max_ctx, q_lens, kv.k.dtype,
-                                attn_order)
+    Hq = _q_heads(model, kv)
+    layer_attn = LayerAttention(kv, rows, B, T, Hq, max_ctx, q_lens, kv.k.dtype, attn_order)
+    layers, consts = [], []
     for layer in inner.layers:
-        attn = layer.self_attn
+        sub = layer._modules  # (nn.Module's attribute lookup costs a microsecond each)
+        attn, mlp = sub["self_attn"], sub["mlp"]
         if getattr(attn, "sliding_window", None) is not None:
             raise NotImplementedError("sliding-window attention needs a windowed mask; this model uses it")
-        li = attn.layer_idx
-        norm = layer.input_layernorm
-        mlp = layer.mlp
-        q = kernels.fused_qkv(residual, norm.weight, norm.variance_epsilon,
-                              attn.qkv_weight_blk if blk else attn.qkv_weight, attn.qkv_bias, cos,
-                              sin, kv.k[li], kv.v[li], kv.tables, kv.lens,
-                              attn.num_key_value_groups * kv.k.shape[2], seq_rows=rows,
-                              q_lens=q_lens, blocked_w=blk)
-        out = layer_attn(q, li, attn.scaling)
-        kernels.linear_residual(out.view(B * T, -1), attn.o_weight_blk if blk else attn.o_proj.weight,
-                                residual, blocked_w=blk)
-        post = layer.post_attention_layernorm
-        act = kernels.fused_gate_up(residual, post.weight, post.variance_epsilon,
-                                    mlp.gate_up_weight_blk if blk else mlp.gate_up_weight,
-                                    blocked_w=blk)
-        kernels.linear_residual(act, mlp.down_weight_blk if blk else mlp.down_proj.weight, residual,
-                                blocked_w=blk)
-    return kernels.rmsnorm(residual, inner.norm.weight, inner.norm.variance_epsilon)
+        norm, post = sub["input_layernorm"], sub["post_attention_layernorm"]
+        layers.append((attn.layer_idx, norm.weight, attn.qkv_weight_blk if blk else attn.qkv_weight,
+                       attn.qkv_bias, attn.o_weight_blk if blk else attn.o_proj.weight, post.weight,
+                       mlp.gate_up_weight_blk if blk else mlp.gate_up_weight,
+                       mlp.down_weight_blk if blk else mlp.down_proj.weight))
+        consts.append((norm.variance_epsilon, post.variance_epsilon, attn.scaling))
+    return kernels.small_pass(layers, consts, residual, cos, sin, kv, rows, q_lens, Hq,
+                              layer_attn.plan, max_ctx, attn_order, inner.norm.weight,
+                              inner.norm.variance_epsilon, blk)
 
 
 # The split-K layer hands its projections blocked activations (16-row x

@@ -10,6 +10,8 @@ captured with it stays valid after a later launch grows the cache.
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -546,6 +548,65 @@ def fused_gate_up(residual: torch.Tensor, norm_weight: torch.Tensor, eps: float,
                                       _stream(residual.device))
     _lib.check(rc, "kve_fused_gate_up")
     return act
+
+
+def small_pass(layers: list, consts: list, residual: torch.Tensor, cos: torch.Tensor,
+               sin: torch.Tensor, kv, rows: torch.Tensor, q_lens: torch.Tensor | None,
+               num_q_heads: int, plan: AttnPlan, max_ctx: int, attn_order: tuple[int, int],
+               norm_weight: torch.Tensor, eps: float, blocked_w: bool) -> torch.Tensor:
+    """Every layer of a small decode pass in one host call (kve_small_pass):
+    fused_qkv, paged_verify_attn, linear_residual, fused_gate_up and
+    linear_residual per layer, then the final rmsnorm, which is returned.
+    layers: per layer (li, input norm weight, [q|k|v] weight, bias, o_proj
+    weight, post norm weight, [gate|up] weight, down_proj weight), li the pool
+    layer; consts: per layer (input norm eps, post norm eps, softmax scale or
+    None for head_dim ** -0.5).
+    The same checks as those calls make, and residual is updated in place."""
+    dev, bf16 = residual.device, torch.bfloat16
+    _need(residual.dim() == 3 and residual.is_contiguous() and residual.dtype == bf16,
+          "residual must be contiguous bf16 [B, T, H]")
+    B, T, H = residual.shape
+    L, NB, Hkv, bs, D = kv.k.shape
+    _need(tuple(kv.v.shape) == (L, NB, Hkv, D, bs) and kv.k[0].is_contiguous()
+          and kv.v[0].is_contiguous() and kv.k.dtype == kv.v.dtype == bf16,
+          "pools must be bf16 [L, NB, Hkv, bs, D] with contiguous layers")
+    _need(cos.numel() == B * T * D and sin.shape == cos.shape and cos.is_contiguous()
+          and sin.is_contiguous(), "cos/sin shape")
+    max_blocks, num_rows = _attn_checks(kv.tables, kv.lens, rows, q_lens, B, bs, max_ctx, dev)
+    ub, kw = attn_order
+    _need(plan.key == _attn_key(B, T, num_q_heads, Hkv, D, bs, max_ctx, ub, kw, bf16),
+          "attention plan was built for another shape or configuration")
+    q_dim = num_q_heads * D
+    F = layers[0][6].shape[0] // 2
+    wanted = ((H,), (q_dim + 2 * Hkv * D, H), (q_dim + 2 * Hkv * D,), (H, q_dim), (H,), (2 * F, H),
+              (H, F))
+    kp, k_step, vp, v_step = (kv.k.data_ptr(), 2 * kv.k.stride(0), kv.v.data_ptr(),
+                              2 * kv.v.stride(0))
+    ptrs = []
+    for li, *ws in layers:
+        _need(0 <= li < L, f"layer {li} of a pool of {L}")
+        for w, shape in zip(ws, wanted):
+            _need(w.shape == shape and w.dtype is bf16 and w.is_contiguous(), "layer weight shape")
+        n1, qkv, bias, o, n2, gu, down = ws
+        ptrs += (n1.data_ptr(), qkv.data_ptr(), bias.data_ptr(), kp + li * k_step, vp + li * v_step,
+                 o.data_ptr(), n2.data_ptr(), gu.data_ptr(), down.data_ptr())
+    _need(norm_weight.shape == (H,) and norm_weight.dtype is bf16, "final norm weight")
+    q = torch.empty(2, B * T, q_dim, dtype=bf16, device=dev)
+    att = torch.empty_like(q)
+    act = torch.empty(2, B * T, F, dtype=bf16, device=dev)
+    out = torch.empty_like(residual)
+    nbytes = attn_workspace_bytes(B, T, num_q_heads, Hkv, D, bs, max_ctx, ub, kw, bf16)
+    ws = workspace("attn_partials", nbytes, dev)
+    flat = [D ** -0.5 if c is None else c for cs in consts for c in cs]
+    rc = _lib.lib().kve_small_pass(
+        (ctypes.c_void_p * len(ptrs))(*ptrs), (ctypes.c_float * len(flat))(*flat), len(layers),
+        residual.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(), att.data_ptr(),
+        act.data_ptr(), kv.tables.data_ptr(), rows.data_ptr(), kv.lens.data_ptr(), _ptr(q_lens), B,
+        T, H, F, num_q_heads, Hkv, D, bs, max_blocks, num_rows, NB, int(max_ctx), int(ub), int(kw),
+        plan.buf.data_ptr(), ws.data_ptr(), ws.numel() * ws.element_size(), norm_weight.data_ptr(),
+        float(eps), out.data_ptr(), _layout(blocked_w), _stream(dev))
+    _lib.check(rc, "kve_small_pass")
+    return out
 
 
 # ---- split-K layers (bf16: decode layer up to 64 rows, wide layer up to 160) ----

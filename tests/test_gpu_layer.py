@@ -10,7 +10,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from kvengine_amd import _lib, kernels
+from kvengine_amd import _lib, forward as fwd_mod, kernels
 from kvengine_amd.arch import TINY, TINY128
 from kvengine_amd.decode import greedy_paged
 from kvengine_amd.forward import apply_rope, forward_hidden
@@ -923,3 +923,54 @@ def test_gather_rows_and_scattered_q(gpu_lib, n, R, C):
     assert (out[rest] == 7.0).all()
     for a, b in zip(*pools):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("arch", [TINY, TINY128], ids=["d64", "d128"])
+@pytest.mark.parametrize("B,T,ragged", [(1, 1, False), (3, 2, True), (4, 16, False)])
+def test_small_pass_is_its_launches_one_by_one(gpu_lib, arch, B, T, ragged):
+    """kve_small_pass gives the bits, and the K/V writes, of the same kernels
+    called layer by layer (1 to 64 rows, ragged q_lens, both weight layouts)."""
+    model = build_model(arch, generate_state_dict(arch, seed=9), dtype=torch.bfloat16, device=DEV)
+    ids = torch.randint(0, arch.vocab, (B, T), generator=torch.Generator().manual_seed(B)).to(DEV)
+    q_lens = torch.tensor([T - b % T for b in range(B)], dtype=torch.int32, device=DEV) if ragged else None
+    rows = torch.arange(B, dtype=torch.int32, device=DEV)
+    inner, out = model.model, []
+    has_blk = getattr(inner.layers[0].self_attn, "qkv_weight_blk", None) is not None
+    for blk in ([False, True] if has_blk else [False]):
+        for whole in (True, False):
+            pool = PagedKVCache.for_model(model, num_blocks=4 * B, block_size=16, max_seqs=B)
+            pool.k.zero_(), pool.v.zero_()
+            for b in range(B):
+                s = pool.new_sequence(b)
+                s.reserve(T)
+                assert s.row == b
+            kv = pool.device_kv()
+            r, cos, sin = fwd_mod._prologue(model, ids, kv, rows, T)
+            Hq = fwd_mod._q_heads(model, kv)
+            at = fwd_mod.LayerAttention(kv, rows, B, T, Hq, T, q_lens, kv.k.dtype)
+            layers, consts = [], []
+            for layer in inner.layers:
+                a, m = layer.self_attn, layer.mlp
+                n1, n2 = layer.input_layernorm, layer.post_attention_layernorm
+                ws = ((a.qkv_weight_blk, a.o_weight_blk, m.gate_up_weight_blk, m.down_weight_blk) if blk
+                      else (a.qkv_weight, a.o_proj.weight, m.gate_up_weight, m.down_proj.weight))
+                layers.append((a.layer_idx, n1.weight, ws[0], a.qkv_bias, ws[1], n2.weight, *ws[2:]))
+                consts.append((n1.variance_epsilon, n2.variance_epsilon, a.scaling))
+            if whole:
+                h = kernels.small_pass(layers, consts, r, cos, sin, kv, rows, q_lens, Hq, at.plan, T,
+                                       (0, 0), inner.norm.weight, inner.norm.variance_epsilon, blk)
+            else:
+                for (li, w1, qkv, bias, o, w2, gu, down), (e1, e2, sc) in zip(layers, consts):
+                    q = kernels.fused_qkv(r, w1, e1, qkv, bias, cos, sin, kv.k[li], kv.v[li], kv.tables,
+                                          kv.lens, Hq, seq_rows=rows, q_lens=q_lens, blocked_w=blk)
+                    kernels.linear_residual(at(q, li, sc).view(B * T, -1), o, r, blocked_w=blk)
+                    act = kernels.fused_gate_up(r, w2, e2, gu, blocked_w=blk)
+                    kernels.linear_residual(act, down, r, blocked_w=blk)
+                h = kernels.rmsnorm(r, inner.norm.weight, inner.norm.variance_epsilon)
+            live = torch.ones(B, T, dtype=torch.bool, device=DEV)
+            if ragged:
+                live = torch.arange(T, device=DEV)[None] < q_lens[:, None]
+            out.append((h[live], pool.k.clone(), pool.v.clone()))
+    for other in out[1:]:
+        for x, y in zip(out[0], other):
+            assert torch.equal(x, y)
