@@ -489,6 +489,30 @@ int kve_small_pass(const void* const* layer_ptrs, const float* layer_consts, int
                    size_t workspace_bytes, const void* norm_weight, float norm_eps, void* out,
                    int layout, void* stream);
 
+/*
+ * kve_f32_pass: every layer of an fp32 pass of at most 160 rows in one host call
+ * (forward.py:187-208), the projections as k-slices whose fixed-order sums are
+ * finished by bias + RoPE + K/V write, or by the residual add + RMSNorm; the
+ * final-normed rows go to `out`. A row's result does not depend on the others.
+ * layer_ptrs, layer_consts: as for kve_small_pass, fp32 row-major weights.
+ * residual [rows, hidden] is updated in place; xn [rows, hidden], q and attn_out
+ * [rows, num_q_heads * head_dim] and act [rows, ffn] are scratch; partials:
+ * kve_f32_pass_bytes(...) bytes of scratch. slots: kve_kv_slots of the pass.
+ * hidden % 64 == 0 and <= 2048, ffn % 64 == 0, head_dim 64 or 128.
+ */
+int kve_f32_pass(const void* const* layer_ptrs, const float* layer_consts, int num_layers,
+                 void* residual, const void* cos, const void* sin, const int32_t* slots, void* xn,
+                 void* q, void* attn_out, void* act, void* partials, size_t partials_bytes,
+                 const int32_t* block_tables, const int32_t* seq_rows, const int32_t* start_pos,
+                 const int32_t* q_lens, int num_seqs, int q_len, int hidden, int ffn,
+                 int num_q_heads, int num_kv_heads, int head_dim, int block_size, int max_blocks,
+                 int num_rows, int num_blocks, int max_ctx, int unit_blocks, int key_waves,
+                 const void* plan, void* workspace, size_t workspace_bytes,
+                 const void* norm_weight, float norm_eps, void* out, void* stream);
+
+size_t kve_f32_pass_bytes(int rows, int hidden, int ffn, int num_q_heads, int num_kv_heads,
+                          int head_dim);
+
 #ifdef __cplusplus
 }
 #endif

@@ -46,6 +46,8 @@ EXPORTS = (
     "kve_linear_rows",
     "kve_linear_rows_slices",
     "kve_small_pass",
+    "kve_f32_pass",
+    "kve_f32_pass_bytes",
 )
 
 DTYPE_F32 = 0
@@ -93,6 +95,9 @@ _SIGS = {
     "kve_gate_up_silu": (I, [P, P, P, I, I, I, I, P]),
     "kve_linear_rows": (I, [P, P, P, I, I, I, I, I, P]),
     "kve_linear_rows_slices": (I, [I, I, I, I]),
+    "kve_f32_pass_bytes": (SZ, [I, I, I, I, I, I]),
+    "kve_f32_pass": (I, [P, P, I, P, P, P, P, P, P, P, P, P, SZ, P, P, P, P, I, I, I, I, I, I, I, I, I,
+                         I, I, I, I, I, P, P, SZ, P, F, P, P]),
     "kve_small_pass": (I, [P, P, I, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, I, I, I,
                            I, I, P, P, SZ, P, F, P, I, P]),
 }

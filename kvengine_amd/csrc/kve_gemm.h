@@ -89,7 +89,10 @@ struct DmaGemm {
   // k-step is one contiguous 1 KB block, so an instruction reads two 512-byte
   // runs where the row-major layout gives it eight 128-byte pieces of eight
   // rows. The loads and the LDS image are otherwise the same.
-  template <bool BLK = false, typename WRow, typename After = NoStep>
+  // F32: fp32 matrices read as uint16 pairs (K, xstride, ks0 and ks1 count
+  // uint16: a k-step is 16 values); a lane's fragments hold four consecutive k
+  // of their row, multiplied by four 16x16x4 MFMAs.
+  template <bool BLK = false, bool F32 = false, typename WRow, typename After = NoStep>
   __device__ __forceinline__ static void run(const uint16_t* w, WRow wrow, const uint16_t* x,
                                              int64_t xstride, int M, int K, int ks0, int ks1,
                                              uint16_t* lds, f32x4 (&acc)[WN][MTW],
@@ -154,7 +157,16 @@ struct DmaGemm {
 #pragma unroll
         for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
-          for (int j = 0; j < WN; ++j) acc[j][mt] = mfma16x16x32_bf16(av[j], fb[cur][mt], acc[j][mt]);
+          for (int j = 0; j < WN; ++j) {
+            if constexpr (F32) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                acc[j][mt] = mfma16x16x4_f32(__uint_as_float(av[j][e]), __uint_as_float(fb[cur][mt][e]),
+                                             acc[j][mt]);
+            } else {
+              acc[j][mt] = mfma16x16x32_bf16(av[j], fb[cur][mt], acc[j][mt]);
+            }
+          }
         if (live) after(c0 + kk);
       }
     };

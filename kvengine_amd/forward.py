@@ -225,6 +225,8 @@ def forward_hidden(model, input_ids: torch.Tensor, kv: DeviceKV, rows: torch.Ten
         if _wide_ok(model, n):
             return _forward_splitk(model, input_ids, kv, rows, max_ctx, q_lens, attn_order, wide=True,
                                    blocked_out=blocked_out)
+        if _f32_ok(model, n):
+            return _forward_f32(model, input_ids, kv, rows, max_ctx, q_lens, attn_order)
         return _forward_fused(model, input_ids, kv, rows, max_ctx, q_lens, attn_order)
     inner = model.model
     B, T = input_ids.shape
@@ -522,8 +524,17 @@ def _forward_small(model, input_ids, kv: DeviceKV, rows, max_ctx, q_lens, attn_o
     residual, cos, sin = _prologue(model, input_ids, kv, rows, max_ctx)
     Hq = _q_heads(model, kv)
     layer_attn = LayerAttention(kv, rows, B, T, Hq, max_ctx, q_lens, kv.k.dtype, attn_order)
+    layers, consts = _pass_layers(model, blk)
+    return kernels.small_pass(layers, consts, residual, cos, sin, kv, rows, q_lens, Hq,
+                              layer_attn.plan, max_ctx, attn_order, inner.norm.weight,
+                              inner.norm.variance_epsilon, blk)
+
+
+def _pass_layers(model, blk: bool = False):
+    """Per layer the operands and the constants of a whole-pass call
+    (kernels.small_pass); blk: the blocked weight copies."""
     layers, consts = [], []
-    for layer in inner.layers:
+    for layer in model.model.layers:
         sub = layer._modules  # (nn.Module's attribute lookup costs a microsecond each)
         attn, mlp = sub["self_attn"], sub["mlp"]
         if getattr(attn, "sliding_window", None) is not None:
@@ -534,9 +545,41 @@ def _forward_small(model, input_ids, kv: DeviceKV, rows, max_ctx, q_lens, attn_o
                        mlp.gate_up_weight_blk if blk else mlp.gate_up_weight,
                        mlp.down_weight_blk if blk else mlp.down_proj.weight))
         consts.append((norm.variance_epsilon, post.variance_epsilon, attn.scaling))
-    return kernels.small_pass(layers, consts, residual, cos, sin, kv, rows, q_lens, Hq,
-                              layer_attn.plan, max_ctx, attn_order, inner.norm.weight,
-                              inner.norm.variance_epsilon, blk)
+    return layers, consts
+
+
+def _f32_ok(model, rows: int) -> bool:
+    """kve_f32_pass takes this model's layers and this many rows."""
+    if not SMALL_BATCH_FUSION or rows > kernels.F32_PASS_ROWS:
+        return False
+    layer = model.model.layers[0]
+    a, mlp = layer.self_attn, layer.mlp
+    if a.qkv_weight.dtype != torch.float32 or a.qkv_bias is None or a.o_proj.bias is not None \
+            or mlp.down_proj.bias is not None or a.head_dim not in (64, 128):
+        return False
+    H, F = mlp.down_proj.weight.shape
+    return H % 64 == 0 and H <= 2048 and F % 64 == 0
+
+
+def _forward_f32(model, input_ids, kv: DeviceKV, rows, max_ctx, q_lens, attn_order):
+    """The fp32 layer of at most 160 rows, issued by one host call: per layer
+    q/k/v k-slices, their sum + bias + RoPE + KV write, attention (+ its split
+    merge), o_proj k-slices, their sum + residual + RMSNorm, gate/up + SiLU*up,
+    down_proj k-slices, their sum + residual + the next RMSNorm (0.5B at 20
+    rows, 4 layers: 718 us as library GEMMs and separate launches)."""
+    inner = model.model
+    B, T = input_ids.shape
+    residual, cos, sin = _prologue(model, input_ids, kv, rows, max_ctx)
+    Hq = _q_heads(model, kv)
+    layer_attn = LayerAttention(kv, rows, B, T, Hq, max_ctx, q_lens, kv.k.dtype, attn_order)
+    layers, consts = _pass_layers(model)
+    # weights that the library GEMMs took as they are and the kernels cannot read
+    layers = [(li, *(w if w.is_contiguous() and w.data_ptr() % 16 == 0
+                     else w.clone(memory_format=torch.contiguous_format) for w in ws))
+              for li, *ws in layers]
+    return kernels.f32_pass(layers, consts, residual, cos, sin, kv, rows, q_lens, Hq,
+                            layer_attn.plan, max_ctx, attn_order, inner.norm.weight,
+                            inner.norm.variance_epsilon)
 
 
 # The split-K layer hands its projections blocked activations (16-row x

@@ -429,7 +429,8 @@ def pass_prologue(ids: torch.Tensor, embed: torch.Tensor, lens: torch.Tensor, se
     B, T = ids.shape
     V, H = embed.shape
     P, D = cos_table.shape
-    _need(embed.dtype == cos_table.dtype == sin_table.dtype == torch.bfloat16, "bf16 tables")
+    _need(embed.dtype == cos_table.dtype == sin_table.dtype
+          and embed.dtype in (torch.bfloat16, torch.float32), "bf16 or fp32 tables of one dtype")
     _need(embed.is_contiguous() and cos_table.is_contiguous() and sin_table.is_contiguous()
           and tuple(sin_table.shape) == (P, D), "contiguous embedding and RoPE tables")
     _check_i32(lens, "lens", dev)
@@ -439,10 +440,12 @@ def pass_prologue(ids: torch.Tensor, embed: torch.Tensor, lens: torch.Tensor, se
     cos = torch.empty(B, T, D, dtype=embed.dtype, device=dev)
     sin = torch.empty(B, T, D, dtype=embed.dtype, device=dev)
     _need(lens.numel() > 0, "lens must hold at least one table row")
-    rc = _lib.lib().kve_pass_prologue(ids.data_ptr(), embed.data_ptr(), V, H, lens.data_ptr(),
+    # the kernel copies rows of 2-byte values; an fp32 row is one of twice as many
+    e = embed.element_size() // 2
+    rc = _lib.lib().kve_pass_prologue(ids.data_ptr(), embed.data_ptr(), V, e * H, lens.data_ptr(),
                                       seq_rows.data_ptr(), lens.numel(), B, T, cos_table.data_ptr(),
-                                      sin_table.data_ptr(), P, D, hidden.data_ptr(), cos.data_ptr(),
-                                      sin.data_ptr(), _stream(dev))
+                                      sin_table.data_ptr(), P, e * D, hidden.data_ptr(),
+                                      cos.data_ptr(), sin.data_ptr(), _stream(dev))
     _lib.check(rc, "kve_pass_prologue")
     return hidden, cos, sin
 
@@ -550,6 +553,45 @@ def fused_gate_up(residual: torch.Tensor, norm_weight: torch.Tensor, eps: float,
     return act
 
 
+def _pass_operands(layers: list, consts: list, residual, cos, sin, kv, rows, q_lens, Hq: int,
+                   plan: AttnPlan, max_ctx: int, order: tuple[int, int], norm_weight, dtype):
+    """Checks the operands of a whole-pass call (small_pass, f32_pass) as the
+    single launches check theirs; returns the layers' pointer and constant
+    arrays, the ffn width, the table's (max_blocks, rows) and the attention
+    workspace."""
+    _need(residual.dim() == 3 and residual.is_contiguous() and residual.dtype is dtype,
+          f"residual must be contiguous {dtype} [B, T, H]")
+    B, T, H = residual.shape
+    L, NB, Hkv, bs, D = kv.k.shape
+    _need(tuple(kv.v.shape) == (L, NB, Hkv, D, bs) and kv.k[0].is_contiguous()
+          and kv.v[0].is_contiguous() and kv.k.dtype == kv.v.dtype == dtype,
+          f"pools must be {dtype} [L, NB, Hkv, bs, D] with contiguous layers")
+    _need(cos.numel() == B * T * D and sin.shape == cos.shape and cos.is_contiguous()
+          and sin.is_contiguous() and cos.dtype == sin.dtype == dtype, "cos/sin shape")
+    tables = _attn_checks(kv.tables, kv.lens, rows, q_lens, B, bs, max_ctx, residual.device)
+    _need(plan.key == _attn_key(B, T, Hq, Hkv, D, bs, max_ctx, *order, dtype),
+          "attention plan was built for another shape or configuration")
+    q_dim, F = Hq * D, layers[0][6].shape[0] // 2
+    wanted = ((H,), (q_dim + 2 * Hkv * D, H), (q_dim + 2 * Hkv * D,), (H, q_dim), (H,), (2 * F, H),
+              (H, F))
+    e = residual.element_size()
+    kp, k_step, vp, v_step = (kv.k.data_ptr(), e * kv.k.stride(0), kv.v.data_ptr(),
+                              e * kv.v.stride(0))
+    ptrs = []
+    for li, *ws in layers:
+        _need(0 <= li < L, f"layer {li} of a pool of {L}")
+        for w, shape in zip(ws, wanted):
+            _need(w.shape == shape and w.dtype is dtype and w.is_contiguous(), "layer weight shape")
+        n1, qkv, bias, o, n2, gu, down = ws
+        ptrs += (n1.data_ptr(), qkv.data_ptr(), bias.data_ptr(), kp + li * k_step, vp + li * v_step,
+                 o.data_ptr(), n2.data_ptr(), gu.data_ptr(), down.data_ptr())
+    _need(norm_weight.shape == (H,) and norm_weight.dtype is dtype, "final norm weight")
+    flat = [D ** -0.5 if c is None else c for cs in consts for c in cs]
+    nbytes = attn_workspace_bytes(B, T, Hq, Hkv, D, bs, max_ctx, *order, dtype)
+    return ((ctypes.c_void_p * len(ptrs))(*ptrs), (ctypes.c_float * len(flat))(*flat), F, tables,
+            workspace("attn_partials", nbytes, residual.device))
+
+
 def small_pass(layers: list, consts: list, residual: torch.Tensor, cos: torch.Tensor,
                sin: torch.Tensor, kv, rows: torch.Tensor, q_lens: torch.Tensor | None,
                num_q_heads: int, plan: AttnPlan, max_ctx: int, attn_order: tuple[int, int],
@@ -560,52 +602,60 @@ def small_pass(layers: list, consts: list, residual: torch.Tensor, cos: torch.Te
     layers: per layer (li, input norm weight, [q|k|v] weight, bias, o_proj
     weight, post norm weight, [gate|up] weight, down_proj weight), li the pool
     layer; consts: per layer (input norm eps, post norm eps, softmax scale or
-    None for head_dim ** -0.5).
-    The same checks as those calls make, and residual is updated in place."""
+    None for head_dim ** -0.5). residual is updated in place."""
     dev, bf16 = residual.device, torch.bfloat16
-    _need(residual.dim() == 3 and residual.is_contiguous() and residual.dtype == bf16,
-          "residual must be contiguous bf16 [B, T, H]")
+    ptrs, flat, F, (max_blocks, num_rows), ws = _pass_operands(
+        layers, consts, residual, cos, sin, kv, rows, q_lens, num_q_heads, plan, max_ctx, attn_order,
+        norm_weight, bf16)
     B, T, H = residual.shape
-    L, NB, Hkv, bs, D = kv.k.shape
-    _need(tuple(kv.v.shape) == (L, NB, Hkv, D, bs) and kv.k[0].is_contiguous()
-          and kv.v[0].is_contiguous() and kv.k.dtype == kv.v.dtype == bf16,
-          "pools must be bf16 [L, NB, Hkv, bs, D] with contiguous layers")
-    _need(cos.numel() == B * T * D and sin.shape == cos.shape and cos.is_contiguous()
-          and sin.is_contiguous(), "cos/sin shape")
-    max_blocks, num_rows = _attn_checks(kv.tables, kv.lens, rows, q_lens, B, bs, max_ctx, dev)
-    ub, kw = attn_order
-    _need(plan.key == _attn_key(B, T, num_q_heads, Hkv, D, bs, max_ctx, ub, kw, bf16),
-          "attention plan was built for another shape or configuration")
-    q_dim = num_q_heads * D
-    F = layers[0][6].shape[0] // 2
-    wanted = ((H,), (q_dim + 2 * Hkv * D, H), (q_dim + 2 * Hkv * D,), (H, q_dim), (H,), (2 * F, H),
-              (H, F))
-    kp, k_step, vp, v_step = (kv.k.data_ptr(), 2 * kv.k.stride(0), kv.v.data_ptr(),
-                              2 * kv.v.stride(0))
-    ptrs = []
-    for li, *ws in layers:
-        _need(0 <= li < L, f"layer {li} of a pool of {L}")
-        for w, shape in zip(ws, wanted):
-            _need(w.shape == shape and w.dtype is bf16 and w.is_contiguous(), "layer weight shape")
-        n1, qkv, bias, o, n2, gu, down = ws
-        ptrs += (n1.data_ptr(), qkv.data_ptr(), bias.data_ptr(), kp + li * k_step, vp + li * v_step,
-                 o.data_ptr(), n2.data_ptr(), gu.data_ptr(), down.data_ptr())
-    _need(norm_weight.shape == (H,) and norm_weight.dtype is bf16, "final norm weight")
-    q = torch.empty(2, B * T, q_dim, dtype=bf16, device=dev)
+    _, NB, Hkv, bs, D = kv.k.shape
+    q = torch.empty(2, B * T, num_q_heads * D, dtype=bf16, device=dev)
     att = torch.empty_like(q)
     act = torch.empty(2, B * T, F, dtype=bf16, device=dev)
     out = torch.empty_like(residual)
-    nbytes = attn_workspace_bytes(B, T, num_q_heads, Hkv, D, bs, max_ctx, ub, kw, bf16)
-    ws = workspace("attn_partials", nbytes, dev)
-    flat = [D ** -0.5 if c is None else c for cs in consts for c in cs]
     rc = _lib.lib().kve_small_pass(
-        (ctypes.c_void_p * len(ptrs))(*ptrs), (ctypes.c_float * len(flat))(*flat), len(layers),
-        residual.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(), att.data_ptr(),
-        act.data_ptr(), kv.tables.data_ptr(), rows.data_ptr(), kv.lens.data_ptr(), _ptr(q_lens), B,
-        T, H, F, num_q_heads, Hkv, D, bs, max_blocks, num_rows, NB, int(max_ctx), int(ub), int(kw),
-        plan.buf.data_ptr(), ws.data_ptr(), ws.numel() * ws.element_size(), norm_weight.data_ptr(),
-        float(eps), out.data_ptr(), _layout(blocked_w), _stream(dev))
+        ptrs, flat, len(layers), residual.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(),
+        att.data_ptr(), act.data_ptr(), kv.tables.data_ptr(), rows.data_ptr(), kv.lens.data_ptr(),
+        _ptr(q_lens), B, T, H, F, num_q_heads, Hkv, D, bs, max_blocks, num_rows, NB, int(max_ctx),
+        int(attn_order[0]), int(attn_order[1]), plan.buf.data_ptr(), ws.data_ptr(),
+        ws.numel() * ws.element_size(), norm_weight.data_ptr(), float(eps), out.data_ptr(),
+        _layout(blocked_w), _stream(dev))
     _lib.check(rc, "kve_small_pass")
+    return out
+
+
+F32_PASS_ROWS = 160  # most rows of kve_f32_pass
+
+
+def f32_pass(layers: list, consts: list, residual: torch.Tensor, cos: torch.Tensor,
+             sin: torch.Tensor, kv, rows: torch.Tensor, q_lens: torch.Tensor | None,
+             num_q_heads: int, plan: AttnPlan, max_ctx: int, attn_order: tuple[int, int],
+             norm_weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """Every layer of an fp32 pass (<= F32_PASS_ROWS rows) in one host call
+    (kve_f32_pass), arguments as small_pass with row-major weights."""
+    dev, f32 = residual.device, torch.float32
+    ptrs, flat, F, (max_blocks, num_rows), ws = _pass_operands(
+        layers, consts, residual, cos, sin, kv, rows, q_lens, num_q_heads, plan, max_ctx, attn_order,
+        norm_weight, f32)
+    B, T, H = residual.shape
+    _, NB, Hkv, bs, D = kv.k.shape
+    lib = _lib.lib()
+    slots = kv_slots(kv.tables, kv.lens, B, T, bs, NB, seq_rows=rows, q_lens=q_lens)
+    q = torch.empty(B * T, num_q_heads * D, dtype=f32, device=dev)
+    att = torch.empty_like(q)
+    act = torch.empty(B * T, F, dtype=f32, device=dev)
+    xn, out = torch.empty_like(residual), torch.empty_like(residual)
+    part = torch.empty(lib.kve_f32_pass_bytes(B * T, H, F, num_q_heads, Hkv, D), dtype=torch.uint8,
+                       device=dev)
+    rc = lib.kve_f32_pass(
+        ptrs, flat, len(layers), residual.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+        slots.data_ptr(), xn.data_ptr(), q.data_ptr(), att.data_ptr(), act.data_ptr(),
+        part.data_ptr(), part.numel(), kv.tables.data_ptr(), rows.data_ptr(), kv.lens.data_ptr(),
+        _ptr(q_lens), B, T, H, F, num_q_heads, Hkv, D, bs, max_blocks, num_rows, NB, int(max_ctx),
+        int(attn_order[0]), int(attn_order[1]), plan.buf.data_ptr(), ws.data_ptr(),
+        ws.numel() * ws.element_size(), norm_weight.data_ptr(), float(eps), out.data_ptr(),
+        _stream(dev))
+    _lib.check(rc, "kve_f32_pass")
     return out
 
 

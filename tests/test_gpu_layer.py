@@ -974,3 +974,49 @@ def test_small_pass_is_its_launches_one_by_one(gpu_lib, arch, B, T, ragged):
     for other in out[1:]:
         for x, y in zip(out[0], other):
             assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("arch", [TINY, TINY128], ids=["d64", "d128"])
+@pytest.mark.parametrize("B,T,ragged", [(1, 1, False), (16, 1, False), (17, 1, False), (3, 7, True),
+                                        (16, 5, True), (8, 20, False)])
+def test_f32_pass_matches_the_library_layer(gpu_lib, arch, B, T, ragged, monkeypatch):
+    """kve_f32_pass (1 to 160 rows, ragged) against the layer of library GEMMs
+    over the same histories. Both sum in fp32 in different orders: a dot product
+    of K terms moves by about sqrt(K) 2^-24 (ffn <= 512: 1.4e-6) of its size, and
+    the layers add up; 2e-5 of the largest value allows for each. Rows past q_len
+    write nothing, and a sequence alone gets the bits it gets in the batch."""
+    model = build_model(arch, generate_state_dict(arch, seed=5, dtype=torch.float32),
+                        dtype=torch.float32, device=DEV)
+    assert fwd_mod._f32_ok(model, B * T)
+    g = torch.Generator().manual_seed(B + T)
+    ids = torch.randint(0, arch.vocab, (B, T), generator=g).to(DEV)
+    q_lens = torch.tensor([T - b % T for b in range(B)], dtype=torch.int32, device=DEV) if ragged else None
+    hist = [1 + 13 * b % 40 for b in range(B)]
+
+    def run(rows_of, fuse):
+        monkeypatch.setattr(fwd_mod, "SMALL_BATCH_FUSION", fuse)
+        pool = PagedKVCache.for_model(model, num_blocks=5 * B + 4, block_size=16, max_seqs=B)
+        for b in range(B):
+            s = pool.new_sequence(b)
+            s.reserve(hist[b] + T)
+            assert s.row == b
+        gk = torch.Generator().manual_seed(7)
+        pool.k.copy_(torch.randn(pool.k.shape, generator=gk))
+        pool.v.copy_(torch.randn(pool.v.shape, generator=gk))
+        pool.lens[:B] = torch.tensor(hist, dtype=torch.int32)
+        rows = torch.tensor(rows_of, dtype=torch.int32, device=DEV)
+        h = forward_hidden(model, ids[rows_of], pool.device_kv(), rows, max(hist) + T,
+                           q_lens=None if q_lens is None else q_lens[rows_of].contiguous(),
+                           attn_order=(8, 1))
+        return h, pool.k.clone(), pool.v.clone()
+
+    everyone = list(range(B))
+    got, want = run(everyone, True), run(everyone, False)
+    live = torch.ones(B, T, dtype=torch.bool, device=DEV)
+    if ragged:
+        live = torch.arange(T, device=DEV)[None] < q_lens[:, None]
+    for x, y in ((got[0][live], want[0][live]), got[1:2] + want[1:2], got[2:] + want[2:]):
+        assert (x - y).abs().max() <= 2e-5 * y.abs().max()
+    alone = run([B - 1], True)[0]
+    n = T if q_lens is None else int(q_lens[B - 1])
+    assert torch.equal(alone[0, :n], got[0][B - 1, :n])
