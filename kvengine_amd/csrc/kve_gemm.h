@@ -4,6 +4,8 @@
 
 #include "kve_common.h"
 
+#include <type_traits>
+
 namespace kve {
 
 // s_waitcnt immediate: at most n vector-memory operations and no LDS operation
@@ -181,6 +183,118 @@ struct DmaGemm {
       compute(lds + static_cast<size_t>(c % NBUF) * (CH_BYTES / 2), ks0 + c * KC);
     }
     __syncthreads();  // the caller may reuse the LDS once every wave is done
+  }
+};
+
+// The same product (operands, lanes, k order, acc layout and arguments of
+// DmaGemm::run, so the same bits) for row counts where the CUs have work to
+// overlap: every k-step has an LDS buffer of its own (NB of them, NB - 1 in
+// flight), and its fragments are read, and a later k-step's loads issued, in
+// between the MFMAs of the k-step before (the scheduling barriers hold every
+// read and load at its place). One barrier per k-step, no LDS latency in front
+// of the MFMAs. A buffer is 1 KB pieces of 16 rows x 32 columns, one direct
+// load each, their 16-byte units swizzled so that the 16 rows of a fragment
+// read fall in different bank groups. Meant for two workgroups per CU (<= 80 KB,
+// <= 256 registers on 4 waves): one multiplies while the other waits at its
+// barrier, loads its first k-steps or writes its outputs.
+template <int MT, int NW, int WN, int NB, int NR>
+struct StepGemm {
+  static constexpr int NC = NW / NR, MTW = MT / NR;
+  static_assert(NC * NR == NW && MTW * NR == MT && NB >= 3, "waves split evenly into row groups");
+  static constexpr int BN = 16 * WN * NC, XROWS = 16 * MT;
+  static constexpr int NT = 64 * NW;
+  static constexpr int PIECES = WN * NC + MT;           // 1 KB pieces of a k-step
+  static constexpr int U = (PIECES + NW - 1) / NW;      // of which each wave loads U
+  static constexpr int BUF = PIECES * 512;              // elements of a buffer
+  static constexpr size_t LDS_BYTES = static_cast<size_t>(NB) * BUF * 2;
+  static_assert((NB - 2) * U <= 63, "vmcnt range");
+
+  struct NoStep {
+    __device__ __forceinline__ void operator()(int) const {}
+  };
+
+  template <bool BLK = false, typename WRow, typename After = NoStep>
+  __device__ __forceinline__ static void run(const uint16_t* w, WRow wrow, const uint16_t* x,
+                                             int64_t xstride, int M, int K, int ks0, int ks1,
+                                             uint16_t* lds, f32x4 (&acc)[WN][MTW],
+                                             After after = After{}) {
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wc = wv % NC, wr = wv / NC;
+    const int l = threadIdx.x & 63, lr = l & 15, lg = l >> 4;
+    // this wave's pieces NW i + wv (the last one again past PIECES: the same
+    // bytes to the same place): lane l fills 16-byte unit l with unit c of row r
+    const uint16_t* src[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const int t = min(NW * i + wv, PIECES - 1);
+      const int r = l >> 2, c = (l & 3) ^ ((r >> 2) & 3);
+      if (t < BN / 16) {
+        src[i] = w + mat_off(wrow(16 * t + r), 8 * c, K, K, BLK);
+      } else {
+        src[i] = x + mat_off(min(16 * (t - BN / 16) + r, M - 1), 8 * c, K, xstride, BLK);
+      }
+    }
+    constexpr int KSTEP = BLK ? 512 : 32;  // elements from one k-step to the next
+    auto dma = [&](int i, int ks, uint16_t* buf) {
+      __builtin_amdgcn_global_load_lds(
+          (__attribute__((address_space(1))) void*)(src[i] + KSTEP * ks),
+          (__attribute__((address_space(3))) void*)(buf + 512 * min(NW * i + wv, PIECES - 1)), 16, 0, 0);
+    };
+    auto rd = [](const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); };
+    const int fo = 8 * (lr * 4 + (lg ^ ((lr >> 2) & 3)));
+    const int ao = WN * wc * 512 + fo, bo = (BN / 16 + MTW * wr) * 512 + fo;
+    // Every load is issued (k-steps past ks1 re-read the last one into buffers
+    // nothing reads), so each wait below is exact.
+#pragma unroll
+    for (int q = 0; q < NB - 1; ++q)
+#pragma unroll
+      for (int i = 0; i < U; ++i) dma(i, min(ks0 + q, ks1 - 1), lds + q * BUF);
+    barrier_after_vm<(NB - 2) * U>();
+    u32x4 fa[2][WN], fb[2][MTW];
+#pragma unroll
+    for (int j = 0; j < WN; ++j) fa[0][j] = rd(lds + ao + 512 * j);
+#pragma unroll
+    for (int mt = 0; mt < MTW; ++mt) fb[0][mt] = rd(lds + bo + 512 * mt);
+#pragma unroll
+    for (int i = 0; i < U; ++i) dma(i, min(ks0 + NB - 1, ks1 - 1), lds + (NB - 1) * BUF);
+
+    auto step = [&](int ks, auto CUR) {
+      constexpr int cur = decltype(CUR)::value, nxt = cur ^ 1;
+      // k-step ks + 1 has landed for every wave, and every wave has read its
+      // fragments of ks, whose buffer takes k-step ks + NB
+      barrier_after_vm<(NB - 2) * U>();
+      const uint16_t* nb = lds + ((ks - ks0 + 1) % NB) * BUF;
+      uint16_t* db = lds + ((ks - ks0) % NB) * BUF;
+      const int dk = min(ks + NB, ks1 - 1);
+      // SLOTS fragment reads and loads, evenly over the first 85 % of the MFMAs
+      constexpr int MF = WN * MTW, SLOTS = WN + MTW + U;
+      auto slot = [&](int o) {
+        const int a = o * U / SLOTS;  // loads before this slot
+        if ((o + 1) * U / SLOTS > a) dma(a, dk, db);
+        else if (o - a < MTW) fb[nxt][o - a] = rd(nb + bo + 512 * (o - a));
+        else fa[nxt][o - a - MTW] = rd(nb + ao + 512 * (o - a - MTW));
+      };
+      int o = 0;
+#pragma unroll
+      for (int q = 0; q < MF; ++q) {
+        const int j = q / MTW, mt = q % MTW;
+        acc[j][mt] = mfma16x16x32_bf16(fa[cur][j], fb[cur][mt], acc[j][mt]);
+        const int want = q + 1 == MF ? SLOTS : min(SLOTS, (q + 1) * SLOTS * 100 / (MF * 85));
+        if (o < want) {
+          __builtin_amdgcn_sched_barrier(0);
+          for (; o < want; ++o) slot(o);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      after(ks);
+    };
+    int ks = ks0;
+    for (; ks + 1 < ks1; ks += 2) {
+      step(ks, std::integral_constant<int, 0>{});
+      step(ks + 1, std::integral_constant<int, 1>{});
+    }
+    if (ks < ks1) step(ks, std::integral_constant<int, 0>{});
+    barrier_after_vm<0>();  // no load is left; the caller may reuse the LDS
   }
 };
 

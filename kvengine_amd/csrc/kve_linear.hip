@@ -1099,18 +1099,10 @@ __global__ __launch_bounds__(C::NT) void gate_up_silu_kernel(const uint16_t* xn,
 // on the A side, 8 consecutive k of a k-step per lane group), so each slice
 // sum is the split-K kernel's bit for bit.
 //
-// Tile and pipeline. 4 waves as 2 x 2 groups of 64 weight rows x 16 MTW rows: a
-// 128 x 32 MTW tile in at most 80 KB of LDS and 256 registers, so two
-// workgroups share a CU and one multiplies while the other waits at its
-// barrier, loads its first k-steps or writes its outputs. Each k-step has its
-// own LDS buffer (NB of them, NB - 1 in flight): 16-row x 32-column pieces of
-// 1 KB, one per direct load, their 16-byte units swizzled so the 16 rows of a
-// fragment read fall in different bank groups. A k-step's fragments are read,
-// and a later k-step's loads issued, in between the previous k-step's MFMAs
-// (the scheduling barriers hold every read and load at its place): one barrier
-// per k-step, no LDS latency in front of the MFMAs. Workgroups are dealt to the
-// XCDs in contiguous runs of tiles, 4 row tiles by columns, so the 64 tiles an
-// XCD has in flight share their operands in its L2.
+// Tile: StepGemm on 4 waves as 2 x 2 groups of 64 weight rows x 16 MTW rows, a
+// 128 x 32 MTW tile, two workgroups per CU. Workgroups are dealt to the XCDs in
+// contiguous runs of tiles, 4 row tiles by columns, so the 64 tiles an XCD has
+// in flight share their operands in its L2.
 // Before: a 128 x 256 tile on 16 waves (32 x 64 each), one workgroup per CU,
 // fragments read at the start of each chunk, tiles in launch order. It was
 // bound by LDS (192 bytes of fragments per clock at full MFMA rate, 128 are
@@ -1119,15 +1111,8 @@ __global__ __launch_bounds__(C::NT) void gate_up_silu_kernel(const uint16_t* xn,
 // down 332 -> 261 (836 -> 1064), o 81 -> 63 (637 -> 823); at 3000 rows 338 ->
 // 232, 177 -> 134, 65 -> 33. Measured beside it: a 256 x 256 tile on 8 waves
 // (gate/up 471-497 us at 6154 rows) or on 4 (484-506), one workgroup per CU.
-template <int MTW_, int NB_>
-struct RowsTile {
-  static constexpr int WN = 4, MTW = MTW_, NC = 2, NR = 2, NW = NC * NR, NT = 64 * NW, NB = NB_;
-  static constexpr int BN = 16 * WN * NC, BM = 16 * MTW * NR;
-  static constexpr int PIECES = (BN + BM) / 16;      // 1 KB pieces of a k-step
-  static constexpr int U = cdiv(PIECES, NW);         // of which each wave loads U
-  static constexpr int BUF = PIECES * 512;           // elements of a k-step's buffer
-  static constexpr size_t LDS = static_cast<size_t>(NB) * BUF * 2;
-};
+template <int MTW, int NB>
+using RowsTile = StepGemm<2 * MTW, 4, 4, NB, 2>;
 
 // MODE 0-2 as above, or kRowsSlice (one k-slice per workgroup, blockIdx.y, written
 // as linear_splitk_kernel writes it). tot is kept only where slices are summed.
@@ -1137,8 +1122,7 @@ template <int MODE, typename C, bool BLK>
 __global__ __launch_bounds__(C::NT, 2) void linear_rows_kernel(const uint16_t* x, const uint16_t* w,
                                                                void* out, int M, int N, int K, int S,
                                                                int nx, int ny) {
-  constexpr int WN = C::WN, MTW = C::MTW, HALF = WN / 2, U = C::U, NW = C::NW, NB = C::NB;
-  constexpr int BN = C::BN, BUF = C::BUF;
+  constexpr int WN = C::BN / (16 * C::NC), MTW = C::MTW, HALF = WN / 2, BN = C::BN;
   constexpr bool TOT = MODE < 2;
   extern __shared__ __align__(16) uint16_t sm_lin[];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1155,40 +1139,10 @@ __global__ __launch_bounds__(C::NT, 2) void linear_rows_kernel(const uint16_t* x
     by = y0 + o % h;
     bx = o / h;
   }
-  const int m0 = by * C::BM, Mb = min(C::BM, M - m0);
+  const int m0 = by * C::XROWS, Mb = min(C::XROWS, M - m0);
   const int f0 = bx * (BN / 2), n0 = bx * BN, F = N;  // MODE 2: N is the activation width
   int ka = 0, kb = K / 32;                            // k-steps of this workgroup
   if (MODE == kRowsSlice) split_range(K / 32, S, blockIdx.y, ka, kb);
-
-  // this wave's pieces NW i + wv (the last one again past PIECES: same bytes to
-  // the same place): lane l fills 16-byte unit l, which holds unit c of row r
-  const uint16_t* src[U];
-#pragma unroll
-  for (int i = 0; i < U; ++i) {
-    const int t = min(NW * i + wv, C::PIECES - 1);
-    const int r = l >> 2, c = (l & 3) ^ ((r >> 2) & 3);
-    int row;
-    if (t >= BN / 16) {
-      row = m0 + min(16 * (t - BN / 16) + r, Mb - 1);
-    } else if (MODE == 2) {
-      const int j = t % WN, col = f0 + 16 * (HALF * (t / WN) + j % HALF) + r;
-      row = j < HALF ? col : F + col;
-    } else {
-      row = n0 + 16 * t + r;
-    }
-    src[i] = (t < BN / 16 ? w : x) + mat_off(row, 8 * c, K, K, BLK);
-  }
-  constexpr int KSTEP = BLK ? 512 : 32;  // elements from one k-step to the next
-  auto dma = [&](int i, int ks, uint16_t* buf) {
-    __builtin_amdgcn_global_load_lds(
-        (__attribute__((address_space(1))) void*)(src[i] + KSTEP * ks),
-        (__attribute__((address_space(3))) void*)(buf + 512 * min(NW * i + wv, C::PIECES - 1)), 16, 0,
-        0);
-  };
-  auto rd = [](const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); };
-  const int fo = 8 * (lr * 4 + (lg ^ ((lr >> 2) & 3)));
-  const int ao = WN * wc * 512 + fo, bo = (BN / 16 + MTW * wr) * 512 + fo;
-
   f32x4 acc[WN][MTW], tot[TOT ? WN : 1][TOT ? MTW : 1];
   const float t0 = MODE == 1 ? 0.0f : -0.0f;
 #pragma unroll
@@ -1198,71 +1152,29 @@ __global__ __launch_bounds__(C::NT, 2) void linear_rows_kernel(const uint16_t* x
       acc[j][mt] = f32x4{0, 0, 0, 0};
       if constexpr (TOT) tot[j][mt] = f32x4{t0, t0, t0, t0};
     }
-  // Every load is issued (k-steps past kb re-read the last one into buffers
-  // nothing reads), so each wait below is exact.
-#pragma unroll
-  for (int q = 0; q < NB - 1; ++q)
-#pragma unroll
-    for (int i = 0; i < U; ++i) dma(i, min(ka + q, kb - 1), sm_lin + q * BUF);
-  barrier_after_vm<(NB - 2) * U>();
-  u32x4 fa[2][WN], fb[2][MTW];
-#pragma unroll
-  for (int j = 0; j < WN; ++j) fa[0][j] = rd(sm_lin + ao + 512 * j);
-#pragma unroll
-  for (int mt = 0; mt < MTW; ++mt) fb[0][mt] = rd(sm_lin + bo + 512 * mt);
-#pragma unroll
-  for (int i = 0; i < U; ++i) dma(i, min(ka + NB - 1, kb - 1), sm_lin + (NB - 1) * BUF);
-
   int s = 0, next = TOT ? kb / S : 0;  // end of slice 0 (split_range)
-  auto step = [&](int ks, auto CUR) {
-    constexpr int cur = decltype(CUR)::value, nxt = cur ^ 1;
-    // k-step ks + 1 has landed for every wave, and every wave has read its
-    // fragments of ks, whose buffer takes k-step ks + NB
-    barrier_after_vm<(NB - 2) * U>();
-    const uint16_t* nb = sm_lin + ((ks - ka + 1) % NB) * BUF;
-    uint16_t* db = sm_lin + ((ks - ka) % NB) * BUF;
-    const int dk = min(ks + NB, kb - 1);
-    // SLOTS fragment reads and loads, evenly over the first 85 % of the MFMAs
-    constexpr int MF = WN * MTW, SLOTS = WN + MTW + U;
-    auto slot = [&](int o) {
-      const int a = o * U / SLOTS;  // loads before this slot
-      if ((o + 1) * U / SLOTS > a) dma(a, dk, db);
-      else if (o - a < MTW) fb[nxt][o - a] = rd(nb + bo + 512 * (o - a));
-      else fa[nxt][o - a - MTW] = rd(nb + ao + 512 * (o - a - MTW));
-    };
-    int o = 0;
-#pragma unroll
-    for (int q = 0; q < MF; ++q) {
-      const int j = q / MTW, mt = q % MTW;
-      acc[j][mt] = mfma16x16x32_bf16(fa[cur][j], fb[cur][mt], acc[j][mt]);
-      const int want = min(SLOTS, (q + 1) * SLOTS * 100 / (MF * 85));
-      if (o < want) {
-        __builtin_amdgcn_sched_barrier(0);
-        for (; o < want; ++o) slot(o);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
+  auto fold = [&](int ks) {
     if constexpr (TOT) {
-      if (ks + 1 == next) {
+      if (ks + 1 != next) return;
 #pragma unroll
-        for (int j = 0; j < WN; ++j)
+      for (int j = 0; j < WN; ++j)
 #pragma unroll
-          for (int mt = 0; mt < MTW; ++mt) {
-            tot[j][mt] += acc[j][mt];
-            acc[j][mt] = f32x4{0, 0, 0, 0};
-          }
-        ++s;
-        next = static_cast<int>(static_cast<int64_t>(kb) * (s + 1) / S);
-      }
+        for (int mt = 0; mt < MTW; ++mt) {
+          tot[j][mt] += acc[j][mt];
+          acc[j][mt] = f32x4{0, 0, 0, 0};
+        }
+      ++s;
+      next = static_cast<int>(static_cast<int64_t>(kb) * (s + 1) / S);
     }
   };
-  int ks = ka;
-  for (; ks + 1 < kb; ks += 2) {
-    step(ks, std::integral_constant<int, 0>{});
-    step(ks + 1, std::integral_constant<int, 1>{});
-  }
-  if (ks < kb) step(ks, std::integral_constant<int, 0>{});
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));  // no load may land after the wave has ended
+  C::template run<BLK>(
+      w,
+      [f0, n0, F](int r) {
+        if (MODE != 2) return n0 + r;
+        const int t = r >> 4, j = t % WN, col = f0 + 16 * (HALF * (t / WN) + j % HALF) + (r & 15);
+        return j < HALF ? col : F + col;
+      },
+      x + static_cast<size_t>(m0) * K, K, Mb, K, ka, kb, sm_lin, acc, fold);
 
 #pragma unroll
   for (int mt = 0; mt < MTW; ++mt) {
@@ -1855,7 +1767,7 @@ extern "C" int kve_linear_rows(const void* x, const void* weight, void* out, int
   const bool sliced = rows_slices(rows, out_features, in_features, mode) > 1;
   const int N = mode == 2 ? out_features / 2 : out_features;
   const int nx = out_features / unit, cols = sliced ? nx * S : nx;
-  // 256 rows (no room for the running sum) and 160 or 192, else 128
+  // 256 and 192 rows leave no registers for a running sum
   const float c128 = rows_cost(rows, 128, cols), c160 = rows_cost(rows, 160, cols);
   const float c192 = rows_cost(rows, 192, cols), c256 = rows_cost(rows, 256, cols);
   int rc;
@@ -1863,21 +1775,23 @@ extern "C" int kve_linear_rows(const void* x, const void* weight, void* out, int
   do {                                                                                          \
     using C = RowsTile<MTW_, NB_>;                                                              \
     static size_t granted_ = 0, granted_b_ = 0;                                                 \
-    const int ny = cdiv(rows, C::BM);                                                           \
+    const int ny = cdiv(rows, C::XROWS);                                                           \
     const dim3 grid(nx* ny, sliced ? S : 1);                                                    \
     if (blk)                                                                                    \
-      rc = launch_lds(linear_rows_kernel<MODE_, C, true>, granted_b_, grid, dim3(C::NT), C::LDS, st, \
+      rc = launch_lds(linear_rows_kernel<MODE_, C, true>, granted_b_, grid, dim3(C::NT), C::LDS_BYTES, st, \
                       xp, wp, out, rows, N, in_features, S, nx, ny);                            \
     else                                                                                        \
-      rc = launch_lds(linear_rows_kernel<MODE_, C, false>, granted_, grid, dim3(C::NT), C::LDS, st, \
+      rc = launch_lds(linear_rows_kernel<MODE_, C, false>, granted_, grid, dim3(C::NT), C::LDS_BYTES, st, \
                       xp, wp, out, rows, N, in_features, S, nx, ny);                            \
   } while (0)
   if (mode == 2) {
-    if (c256 <= c192 && c256 <= c128) KVE_ROWS(2, 8, 3);
-    else if (c192 <= c128) KVE_ROWS(2, 6, 4);
+    if (c256 <= c192 && c256 <= c160 && c256 <= c128) KVE_ROWS(2, 8, 3);
+    else if (c192 <= c128 && c192 <= c160) KVE_ROWS(2, 6, 4);
+    else if (c160 <= c128) KVE_ROWS(2, 5, 4);
     else KVE_ROWS(2, 4, 4);
   } else if (sliced) {
-    if (c192 <= c128) KVE_ROWS(kRowsSlice, 6, 4);
+    if (c160 <= c128 && c160 <= c192) KVE_ROWS(kRowsSlice, 5, 4);
+    else if (c192 <= c128) KVE_ROWS(kRowsSlice, 6, 4);
     else KVE_ROWS(kRowsSlice, 4, 4);
   } else if (mode == 1) {
     if (c160 <= c128) KVE_ROWS(1, 5, 4);

@@ -166,16 +166,20 @@ __global__ __launch_bounds__(256) void lmhead_argmax_kernel(
 // The hidden rows are staged once per workgroup and shared by its waves, and
 // every tile is read from global memory as whole rows, by direct-to-LDS
 // loads. The keys of the wave columns meet in the dynamic LDS after the GEMM.
-// MINW: waves per SIMD the register allocation must leave room for (2 keeps
-// two 4-wave workgroups on a CU, at most 256 registers per lane).
-template <int MT_, int NW_, int WN_, int KC_, int LDS_, int NR_, int MINW_ = 1>
-struct LmTile {
-  using G = typename DmaCfg<MT_, NW_, WN_, KC_, LDS_, NR_>::G;
+template <typename G_, int MT_, int NW_, int WN_, int NR_, int MINW_>
+struct LmCfg {
+  using G = G_;
   static constexpr int MT = MT_, NW = NW_, WN = WN_, NR = NR_, NC = NW_ / NR_, NT = 64 * NW_;
-  static constexpr int MINW = MINW_;
+  static constexpr int MINW = MINW_;  // waves per SIMD the registers must leave room for
   static constexpr size_t KEY_BYTES = 2 * sizeof(unsigned long long) * NC * 16 * MT_;
   static constexpr size_t LDS = G::LDS_BYTES > KEY_BYTES ? G::LDS_BYTES : KEY_BYTES;
 };
+template <int MT, int NW, int WN, int KC, int LDS, int NR>
+using LmTile = LmCfg<typename DmaCfg<MT, NW, WN, KC, LDS, NR>::G, MT, NW, WN, NR, 1>;
+// 160 embedding rows on 4 waves as 2 x 2, two workgroups per CU (<= 80 KB, <= 256
+// registers)
+template <int MT>
+using LmStep = LmCfg<StepGemm<MT, 4, 5, 4, 2>, MT, 4, 5, 2, 2>;
 
 template <typename C, bool TOP2, bool BLK = false>
 __global__ __launch_bounds__(C::NT, C::MINW) void lmhead_lds_kernel(const uint16_t* hidden, int64_t hstride,
@@ -372,25 +376,29 @@ static int dispatch_lmhead_bf16(int M, const void* hidden, int64_t hs, const voi
                                 const LmOut& o, hipStream_t st, bool blk) {
   const int tiles = cdiv(M, 16);
 #define LM(...) return launch_lmhead_lds<LmTile<__VA_ARGS__>>(hidden, hs, w, M, H, V, o, st, blk)
+#define LM_STEP(MT_)                                                                       \
+  return o.top2() ? launch_lmhead_lds_t<LmStep<MT_>, true, true>(hidden, hs, w, M, H, V, o, st) \
+                  : launch_lmhead_lds_t<LmStep<MT_>, false, true>(hidden, hs, w, M, H, V, o, st)
   if (tiles <= 1) LM(1, 4, 1, 4, 56 * 1024, 1);
   if (tiles <= 2) LM(2, 4, 1, 2, 56 * 1024, 1);
   if (tiles <= 4) LM(4, 4, 1, 2, 56 * 1024, 1);
+  // 65 rows and more, blocked operands: StepGemm over 160 embedding rows. Below,
+  // the embedding's bytes bound the launch and the 64-row tiles stream them at
+  // 5.4-6.2 TB/s; from here the hidden rows that every workgroup reads again
+  // and the chunk waits held the former tiles (DmaGemm, 64 rows on 4 x 1 waves
+  // up to 96 hidden rows, 192 on 2 x 2 above) to 4.1-4.9. 151936 x 2048, HIP
+  // graph, us: 80 rows 124-126 -> 110, 96 131 -> 112, 128 139-148 -> 118, 160
+  // 141-149 -> 125; x 896: 80 rows 55 -> 51, 128 71 -> 58, 160 72 -> 65. 160
+  // embedding rows make 950 workgroups, 1.86 rounds of two per CU: 128 make 2.3
+  // (160 x 2048: 130-136 us) and 192 1.55 (145, and 16 registers spilled).
+  if (blk) {
+    if (tiles <= 6) LM_STEP(6);
+    if (tiles <= 8) LM_STEP(8);
+    LM_STEP(10);
+  }
   if (tiles <= 6) LM(6, 4, 1, 2, 56 * 1024, 1);
-  // 7-10 row tiles, blocked operands: 192 embedding rows on the waves as 2
-  // column x 2 row groups (each wave 6 x 5 tiles) with one-k-step chunks, held
-  // to 256 registers so two workgroups share a CU (240, no spills; without the
-  // bound the compiler takes 294 and one runs per CU: 194 us). Each workgroup
-  // re-reads the hidden rows for 192 embedding rows instead of 128, 19 % fewer
-  // bytes per CU in all: 160 x 2048 x 151936 149.5-150.0 -> 144.3-147.5 us
-  // (HIP graph 156-158 -> 148-150). Earlier: the 4 x 1 split of 128 rows below
-  // takes 260 registers and runs one per CU, 2 x 2 of 128 rows 159 -> 152 us.
-  // Measured no faster: 128- and 256-row tiles on 8 or 10 waves, one
-  // workgroup per CU (163-216 us), three chunk buffers (194 us), 128 rows on 8
-  // waves as 4 x 2 (two per CU: 148.4-148.9 against 149.8-150.3 us) or 10
-  // waves as 2 x 5 (one per CU: 170 us), weight and activation chunks in
-  // separate LDS rings loaded by separate waves (155-157 us).
-  if (blk) LM(10, 4, 6, 1, 72 * 1024, 2, 2);
   LM(10, 4, 2, 2, 56 * 1024, 1);
+#undef LM_STEP
 #undef LM
 }
 

@@ -426,6 +426,14 @@ def forward_packed(model, ids: torch.Tensor, dst: torch.Tensor, B: int, T: int, 
     return h
 
 
+# Gate/up rows above which kve_linear_rows is the faster kernel for the same bits
+# (3B, kve_gate_up_silu / kve_linear_rows: 96 rows 23.8 / 24.6 us, 112 26.0 /
+# 25.1, 128 26.9 / 25.4, 160 29.5 / 27.5; 0.5B: 96 rows 12.0 / 12.5, 112 13.2 /
+# 12.8, 160 15.2 / 12.0). The k-sliced projections are the faster ones, or
+# equal, up to SPLITK_MAX_ROWS (3B down at 96 rows 14.5 / 18.2, at 160 18.8 / 18.8).
+GATE_UP_SILU_ROWS = 104
+
+
 def _wide_proj(x: torch.Tensor, weight: torch.Tensor, mode: int, blocked: bool = False,
                rows: int | None = None) -> torch.Tensor:
     """One projection of the wide split-K layer over any number of rows: k-slice
@@ -435,9 +443,9 @@ def _wide_proj(x: torch.Tensor, weight: torch.Tensor, mode: int, blocked: bool =
     and the gate/up act are blocked matrices (x holding `rows` rows)."""
     if rows is None:
         rows = x.numel() // x.shape[-1]
-    if rows <= SPLITK_MAX_ROWS:
-        if mode == kernels.ROWS_GATE_UP:
-            return kernels.gate_up_silu(x, weight, blocked=blocked, rows=rows)
+    if mode == kernels.ROWS_GATE_UP and rows <= GATE_UP_SILU_ROWS:
+        return kernels.gate_up_silu(x, weight, blocked=blocked, rows=rows)
+    if mode != kernels.ROWS_GATE_UP and rows <= SPLITK_MAX_ROWS:
         return kernels.linear_splitk(x, weight, blocked=blocked, rows=rows)
     return kernels.linear_rows(x, weight, mode, blocked=blocked, rows=rows)
 

@@ -527,3 +527,33 @@ def test_lmhead_runner_up_on_model_like_rows(gpu_lib, M, H, V):
             assert sid[m].item() == top.indices[m, 1].item()
             checked += 1
     assert checked > M // 4
+
+
+@pytest.mark.parametrize("M", [64, 65, 96, 97, 128, 129, 160, 161, 330])
+@pytest.mark.parametrize("H", [96, 256])
+def test_lmhead_blocked_row_tiles_equal_row_major(gpu_lib, M, H):
+    """The blocked LM head at the edges of its row tiles, a vocabulary that is no
+    multiple of its 160-row tiles and an odd count of k-steps: ids, maxima and
+    runner-up of the row-major launch, bit for bit, ties included."""
+    V = 5008
+    g = torch.Generator().manual_seed(M + H)
+    h = torch.randint(-2, 3, (M, H), generator=g).bfloat16().to(DEV)  # many equal logits
+    w = torch.randint(-2, 3, (V, H), generator=g).bfloat16().to(DEV)
+
+    def run(hh, ww, blocked):
+        out = [torch.empty(M, dtype=d, device=DEV) for d in (torch.int32, torch.float32) * 2]
+        kernels.lmhead_argmax(hh, ww, argmax=out[0], maxval=out[1], second_id=out[2],
+                              second_val=out[3], blocked=blocked, rows=M)
+        one = torch.empty(M, dtype=torch.int32, device=DEV)
+        kernels.lmhead_argmax(hh, ww, argmax=one, blocked=blocked, rows=M)
+        assert torch.equal(one, out[0])
+        return out
+
+    want = run(h, w, False)
+    got = run(kernels.to_blocked(h), kernels.to_blocked(w), True)
+    for x, y in zip(got, want):
+        assert torch.equal(x, y)
+    logits = (h.double() @ w.double().T).to(torch.bfloat16).double()
+    top = logits.max(1).values
+    first = torch.where(logits == top[:, None], torch.arange(V, device=DEV), V).min(1).values
+    assert torch.equal(got[0].long(), first) and torch.equal(got[1].double(), top)
