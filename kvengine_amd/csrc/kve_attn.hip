@@ -1137,21 +1137,27 @@ __attribute__((amdgpu_waves_per_eu(NT >= 2 && NT * KW <= 6 ? 4 : 1))) void verif
 
 // Merge the units of one split item (and kv head): the units' states folded
 // in unit order with fold_state -- as the waves of a unit are -- then
-// normalised. Grid (split-item bound, Hkv * D/16); thread (row, 4 channels).
+// normalised. Grid (split-item bound, Hkv * D/16 parts); thread (row, 4 channels).
 // The first two units' states are read before the item's record arrives (its
 // slots follow from its index), the next SPL together once it has, so an item
 // of up to SPL + 2 units costs two round trips; an index past the plan's split
-// items exits.
-template <int D, bool BF16, int NT>
+// items exits. SPL = 16 for launches that latency bounds; 4 for a prefill's
+// many items, which have few units each: with 16, most of a batch's loads
+// re-read the item's last unit. Per launch, with the 64-channel parts: two
+// prompts of 2304 tokens (3B) 67 -> 33 us, one of 1777 (0.5B) 13.7 -> 7.5; the
+// verify shapes' 4.3-8.7 us stay.
+template <int D, bool BF16, int NT, int SPL>
 __global__ __launch_bounds__(64 * NT) void verify_attn_merge_kernel(AttnArgs a) {
   using elem_t = std::conditional_t<BF16, uint16_t, float>;
   constexpr int ROWS = 16 * NT;
-  constexpr int SPL = 16;
   const int tid = threadIdx.x;
   const int j = blockIdx.x;
-  const int kvh = blockIdx.y / (D / 16);
-  const int d = (blockIdx.y - kvh * (D / 16)) * 16 + (tid & 3) * 4;
-  const int rr = tid >> 2;  // < ROWS: the block has 4 * ROWS threads
+  // 64 channels of RPB rows: the part z = 0 .. D/16 - 1 of an item and kv head
+  // (16 channels of every row read 64-byte pieces, half a cache line each)
+  constexpr int CW = 64, LPR = CW / 4, RPB = 64 * NT / LPR, NCB = D / CW;
+  const int kvh = blockIdx.y / (D / 16), z = blockIdx.y - kvh * (D / 16);
+  const int d = (z % NCB) * CW + (tid % LPR) * 4;
+  const int rr = z / NCB * RPB + tid / LPR;  // < ROWS
   const size_t slot0 = static_cast<size_t>(j) * a.max_item_units;
   auto po = [&](int u) {
     return a.part_o + (((slot0 + u) * a.Hkv + kvh) * ROWS + rr) * D + d;
@@ -1381,6 +1387,9 @@ static int launch_plan(const AttnArgs& a, const AttnCfg& p, hipStream_t st) {
   return KVE_OK;
 }
 
+// Merge workgroups from which a launch is bound by its loads (three per CU).
+constexpr long long kMergeMany = 768;
+
 template <int D, bool BF16, int NT, int KW>
 static int launch_attn_t(const AttnArgs& a, const AttnCfg& p, hipStream_t st, bool bs16) {
   auto go = [&](auto kernel) {
@@ -1402,9 +1411,13 @@ static int launch_attn_t(const AttnArgs& a, const AttnCfg& p, hipStream_t st, bo
   if (rc) return rc;
   // histories longer than one unit: merge their units' states (only launched
   // when max_ctx allows more than one unit per history)
-  if (p.max_split > 0)
-    hipLaunchKernelGGL((verify_attn_merge_kernel<D, BF16, NT>), dim3(p.max_split, a.Hkv * (D / 16)),
-                       dim3(64 * NT), 0, st, a);
+  if (p.max_split > 0) {
+    const dim3 grid(p.max_split, a.Hkv * (D / 16));
+    const auto merge = static_cast<long long>(grid.x) * grid.y >= kMergeMany
+                           ? verify_attn_merge_kernel<D, BF16, NT, 4>
+                           : verify_attn_merge_kernel<D, BF16, NT, 16>;
+    hipLaunchKernelGGL(merge, grid, dim3(64 * NT), 0, st, a);
+  }
   return KVE_OK;
 }
 
