@@ -1107,9 +1107,9 @@ __global__ __launch_bounds__(C::NT) void gate_up_silu_kernel(const uint16_t* xn,
 // fragments read at the start of each chunk, tiles in launch order. It was
 // bound by LDS (192 bytes of fragments per clock at full MFMA rate, 128 are
 // served) and by the chunk waits that every wave of the CU shared. 3B layer at
-// 6154 rows, us and TFLOP/s, before -> now: gate/up 664 -> 474 (836 -> 1170),
-// down 332 -> 261 (836 -> 1064), o 81 -> 63 (637 -> 823); at 3000 rows 338 ->
-// 232, 177 -> 134, 65 -> 33. Measured beside it: a 256 x 256 tile on 8 waves
+// 6154 rows, us and TFLOP/s, before -> now: gate/up 647 -> 446 (858 -> 1245),
+// down 332 -> 248 (836 -> 1118), o 78 -> 59 (664 -> 870); at 3000 rows 320 ->
+// 224, 172 -> 134, 64 -> 32. Measured beside it: a 256 x 256 tile on 8 waves
 // (gate/up 471-497 us at 6154 rows) or on 4 (484-506), one workgroup per CU.
 template <int MTW, int NB>
 using RowsTile = StepGemm<2 * MTW, 4, 4, NB, 2>;
