@@ -437,15 +437,18 @@ GATE_UP_SILU_ROWS = 104
 def _wide_proj(x: torch.Tensor, weight: torch.Tensor, mode: int, blocked: bool = False,
                rows: int | None = None) -> torch.Tensor:
     """One projection of the wide split-K layer over any number of rows: k-slice
-    partials [S, rows, out] (or act for gate/up) from the split-K kernels up to
-    SPLITK_MAX_ROWS rows, else the same sums from kve_linear_rows as one slice
-    [1, rows, out]. Either way each row gets the same bits. blocked: x, weight
+    partials [S, rows, out] from kve_linear_splitk up to SPLITK_MAX_ROWS rows and
+    from kve_linear_rows above (every slice, or their sum as [1, rows, out]);
+    gate/up's act from kve_gate_up_silu up to GATE_UP_SILU_ROWS rows, and up to
+    SPLITK_MAX_ROWS for widths that kve_linear_rows does not tile, else from
+    kve_linear_rows. Either way each row gets the same bits. blocked: x, weight
     and the gate/up act are blocked matrices (x holding `rows` rows)."""
     if rows is None:
         rows = x.numel() // x.shape[-1]
-    if mode == kernels.ROWS_GATE_UP and rows <= GATE_UP_SILU_ROWS:
-        return kernels.gate_up_silu(x, weight, blocked=blocked, rows=rows)
-    if mode != kernels.ROWS_GATE_UP and rows <= SPLITK_MAX_ROWS:
+    if mode == kernels.ROWS_GATE_UP:
+        if rows <= GATE_UP_SILU_ROWS or rows <= SPLITK_MAX_ROWS and weight.shape[0] % 128:
+            return kernels.gate_up_silu(x, weight, blocked=blocked, rows=rows)
+    elif rows <= SPLITK_MAX_ROWS:
         return kernels.linear_splitk(x, weight, blocked=blocked, rows=rows)
     return kernels.linear_rows(x, weight, mode, blocked=blocked, rows=rows)
 

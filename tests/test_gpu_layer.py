@@ -6,6 +6,8 @@ in a different order, which may move the float32 result by an ulp and,
 rarely, the rounded model-dtype output by one ulp; that is bounded here.
 """
 
+import dataclasses
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -1020,3 +1022,41 @@ def test_f32_pass_matches_the_library_layer(gpu_lib, arch, B, T, ragged, monkeyp
     alone = run([B - 1], True)[0]
     n = T if q_lens is None else int(q_lens[B - 1])
     assert torch.equal(alone[0, :n], got[0][B - 1, :n])
+
+
+def _histories(model, hist, T, seed=7, blocks=8):
+    """A pool whose sequence b holds hist[b] tokens of seeded K/V, with room for T more."""
+    pool = PagedKVCache.for_model(model, num_blocks=blocks * len(hist) + 4, block_size=16,
+                                  max_seqs=max(len(hist), 1))
+    for b, h in enumerate(hist):
+        s = pool.new_sequence(b)
+        s.reserve(h + T)
+        assert s.row == b
+    g = torch.Generator().manual_seed(seed)
+    pool.k.copy_(torch.randn(pool.k.shape, generator=g))
+    pool.v.copy_(torch.randn(pool.v.shape, generator=g))
+    pool.lens[:len(hist)] = torch.tensor(hist, dtype=torch.int32)
+    return pool
+
+
+@pytest.mark.parametrize("B,T", [(20, 5), (21, 5), (32, 5)])
+def test_gate_up_width_of_32_mod_64(gpu_lib, B, T):
+    """A gate/up width that kve_linear_rows does not tile (2 ffn % 128 != 0) runs
+    at every row count of the wide layer, 100 to 160 rows here, and gives each
+    sequence the bits of a pass of ten sequences."""
+    arch = dataclasses.replace(TINY128, name="ffn288", ffn=288)
+    model = build_model(arch, generate_state_dict(arch, seed=3), dtype=torch.bfloat16, device=DEV)
+    assert fwd_mod._wide_ok(model, B * T) and model.model.layers[0].mlp.gate_up_weight.shape[0] % 128
+    ids = torch.randint(0, arch.vocab, (B, T), generator=torch.Generator().manual_seed(B)).to(DEV)
+    hist = [1 + 7 * b % 40 for b in range(B)]
+
+    def run(seqs):
+        pool = _histories(model, hist, T)
+        rows = torch.tensor(seqs, dtype=torch.int32, device=DEV)
+        return forward_hidden(model, ids[seqs], pool.device_kv(), rows, max(hist) + T,
+                              attn_order=(8, 1), gemm_rows=160)
+
+    whole = run(list(range(B)))
+    for a in range(0, B, 10):
+        part = list(range(a, min(a + 10, B)))
+        assert torch.equal(run(part), whole[part])
