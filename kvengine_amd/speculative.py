@@ -37,7 +37,6 @@ it passes 896 tokens), so a replayed iteration gives the eager iteration's bits.
 
 from __future__ import annotations
 
-import gc
 import time
 import weakref
 from dataclasses import dataclass, field
@@ -145,9 +144,6 @@ class _IterationGraphs:
                tuple(t.data_ptr() for p in (tp, dp) for t in (p.tables, p.lens, p.k, p.v)))
         g = _GRAPHS.get(key)
         if g is None:
-            # dead models' and pools' graphs (kept by reference cycles until a
-            # collection) go now, not while this entry's iterations are captured
-            gc.collect()
             g = _GRAPHS[key] = _IterationGraphs(t_cache.pool, k)
             for obj in (target, draft, t_cache.pool, d_cache.pool):
                 weakref.finalize(obj, _GRAPHS.pop, key, None)

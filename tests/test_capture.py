@@ -3,8 +3,11 @@
 import gc
 import inspect
 import threading
+import weakref
+from types import SimpleNamespace
 
 import pytest
+import torch
 
 from kvengine_amd import engine, speculative
 from kvengine_amd.capture import no_gc
@@ -57,3 +60,42 @@ def test_every_capture_of_the_package_holds_collection_off():
         lines = inspect.getsource(module).splitlines()
         captures = [s for s in lines if "torch.cuda.graph(" in s]
         assert captures and all("no_gc()" in s for s in captures), captures
+
+
+def test_a_new_entry_of_iteration_graphs_collects_nothing(monkeypatch):
+    """A first call on new models and pools, while another thread captures, must
+    not run the collector: what it frees may hold graphs. (A full collection
+    would also cost the call 60-90 ms.)"""
+    class Obj(SimpleNamespace):
+        __hash__ = object.__hash__
+
+    def pool():
+        return Obj(**{n: torch.zeros(1) for n in ("tables", "lens", "k", "v")})
+
+    monkeypatch.setattr(speculative, "_GRAPHS", {})
+    monkeypatch.setattr(speculative._IterationGraphs, "__init__", lambda self, pool, k: None)
+    inside, leave = threading.Event(), threading.Event()
+
+    def capture():
+        with no_gc():
+            inside.set()
+            leave.wait(10)
+
+    t = threading.Thread(target=capture)
+    t.start()
+    assert inside.wait(10)
+    try:
+        dead = Obj()
+        dead.me = dead  # a cycle, as a dead pool's graphs can be in
+        alive = weakref.ref(dead)
+        del dead
+        models = torch.nn.Linear(2, 2), torch.nn.Linear(2, 2)
+        caches = Obj(pool=pool()), Obj(pool=pool())
+        made = speculative._IterationGraphs.for_call(*models, *caches, 4)
+        assert alive() is not None
+        assert speculative._IterationGraphs.for_call(*models, *caches, 4) is made
+    finally:
+        leave.set()
+        t.join()
+    gc.collect()
+    assert alive() is None

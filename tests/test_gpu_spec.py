@@ -11,6 +11,7 @@ from the reference only where the reference's own top-2 logit margin is tiny
 """
 
 import copy
+import gc
 
 import pytest
 import torch
@@ -28,6 +29,13 @@ from kvengine_amd.workloads import OracleAcceptance
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 DTYPES = {"torch.float32": torch.float32, "torch.bfloat16": torch.bfloat16}
+
+
+@pytest.fixture(autouse=True)
+def no_dead_graphs():
+    """Iteration graphs of earlier tests' pools (freed with their reference
+    cycles) leave the table before a test counts its entries, not during it."""
+    gc.collect()
 
 
 class HostileDraft:
