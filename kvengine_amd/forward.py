@@ -222,10 +222,10 @@ def forward_hidden(model, input_ids: torch.Tensor, kv: DeviceKV, rows: torch.Ten
                 return _forward_splitk(model, input_ids, kv, rows, max_ctx, q_lens, attn_order,
                                        blocked_out=blocked_out)
             return _forward_small(model, input_ids, kv, rows, max_ctx, q_lens, attn_order)
-        if _wide_ok(model, n):
+        if _wide_ok(model, n) and (n <= SPLITK_MAX_ROWS or _plain_tokens(model, input_ids)):
             return _forward_splitk(model, input_ids, kv, rows, max_ctx, q_lens, attn_order, wide=True,
                                    blocked_out=blocked_out)
-        if _f32_ok(model, n):
+        if _f32_ok(model, n) and _plain_tokens(model, input_ids):
             return _forward_f32(model, input_ids, kv, rows, max_ctx, q_lens, attn_order)
         return _forward_fused(model, input_ids, kv, rows, max_ctx, q_lens, attn_order)
     inner = model.model
@@ -522,6 +522,15 @@ def _prologue(model, input_ids, kv: DeviceKV, rows, max_ctx):
     emb = inner.embed_tokens.weight
     cos_t, sin_t = inner.rotary_emb.table(emb, max_ctx)
     return kernels.pass_prologue(input_ids, emb, kv.lens, rows, cos_t, sin_t)
+
+
+def _plain_tokens(model, input_ids) -> bool:
+    """_prologue reads these ids and this model's embedding; others (32-bit ids,
+    an embedding at an odd address, strided, or not a plain module) are what
+    embed_tokens itself takes."""
+    emb = model.model.embed_tokens
+    return (input_ids.dtype is torch.int64 and type(emb) is torch.nn.Embedding
+            and emb.weight.is_contiguous() and emb.weight.data_ptr() % 16 == 0)
 
 
 def _forward_small(model, input_ids, kv: DeviceKV, rows, max_ctx, q_lens, attn_order):

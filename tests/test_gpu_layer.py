@@ -1060,3 +1060,36 @@ def test_gate_up_width_of_32_mod_64(gpu_lib, B, T):
     for a in range(0, B, 10):
         part = list(range(a, min(a + 10, B)))
         assert torch.equal(run(part), whole[part])
+
+
+@pytest.mark.parametrize("dtype,T", [(torch.float32, 3), (torch.bfloat16, 200)])
+@pytest.mark.parametrize("what", ["int32 ids", "embedding at an odd address", "strided embedding"])
+def test_tokens_that_the_prologue_kernel_does_not_read(gpu_lib, dtype, T, what, monkeypatch):
+    """Token ids of 32 bits, and an embedding that is not 16-byte aligned or not
+    contiguous, run in the fp32 pass and in prompts of more than 160 tokens as
+    they do with the layer of library GEMMs, and give its bits."""
+    model = build_model(TINY, generate_state_dict(TINY, seed=2, dtype=dtype), dtype=dtype, device=DEV)
+    ids = torch.randint(0, TINY.vocab, (1, T), generator=torch.Generator().manual_seed(T)).to(DEV)
+    rows = torch.zeros(1, dtype=torch.int32, device=DEV)
+    assert fwd_mod._plain_tokens(model, ids)
+
+    def run(i):
+        pool = _histories(model, [5], T, blocks=20)
+        return forward_hidden(model, i, pool.device_kv(), rows, 5 + T), pool.k, pool.v
+
+    monkeypatch.setattr(fwd_mod, "SMALL_BATCH_FUSION", False)
+    want = run(ids)
+    monkeypatch.undo()
+    emb = model.model.embed_tokens
+    w = emb.weight.data
+    if what == "int32 ids":
+        ids = ids.int()
+    elif what == "strided embedding":
+        emb.weight = torch.nn.Parameter(w.t().contiguous().t(), requires_grad=False)
+    else:
+        flat = torch.empty(w.numel() + 1, dtype=dtype, device=DEV)
+        flat[1:] = w.flatten()
+        emb.weight = torch.nn.Parameter(flat[1:].view_as(w), requires_grad=False)
+        assert emb.weight.data_ptr() % 16
+    for x, y in zip(run(ids), want):
+        assert torch.equal(x, y)
