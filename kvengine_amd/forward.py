@@ -589,14 +589,13 @@ def _forward_f32(model, input_ids, kv: DeviceKV, rows, max_ctx, q_lens, attn_ord
     rows, 4 layers: 718 us as library GEMMs and separate launches)."""
     inner = model.model
     B, T = input_ids.shape
+    layers, consts = _pass_layers(model)
+    if not all(w.is_contiguous() and w.data_ptr() % 16 == 0 for _, *ws in layers for w in ws):
+        # the library GEMMs read weights that are strided or at an odd address
+        return _forward_fused(model, input_ids, kv, rows, max_ctx, q_lens, attn_order)
     residual, cos, sin = _prologue(model, input_ids, kv, rows, max_ctx)
     Hq = _q_heads(model, kv)
     layer_attn = LayerAttention(kv, rows, B, T, Hq, max_ctx, q_lens, kv.k.dtype, attn_order)
-    layers, consts = _pass_layers(model)
-    # weights that the library GEMMs took as they are and the kernels cannot read
-    layers = [(li, *(w if w.is_contiguous() and w.data_ptr() % 16 == 0
-                     else w.clone(memory_format=torch.contiguous_format) for w in ws))
-              for li, *ws in layers]
     return kernels.f32_pass(layers, consts, residual, cos, sin, kv, rows, q_lens, Hq,
                             layer_attn.plan, max_ctx, attn_order, inner.norm.weight,
                             inner.norm.variance_epsilon)

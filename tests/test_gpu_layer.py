@@ -1093,3 +1093,31 @@ def test_tokens_that_the_prologue_kernel_does_not_read(gpu_lib, dtype, T, what, 
         assert emb.weight.data_ptr() % 16
     for x, y in zip(run(ids), want):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("which", ["o_proj", "down_proj"])
+@pytest.mark.parametrize("how", ["odd address", "strided"])
+def test_f32_weights_the_pass_does_not_read(gpu_lib, which, how, monkeypatch):
+    """An fp32 model with a projection weight that is not 16-byte aligned or not
+    contiguous takes the layer of library GEMMs, which reads it in place."""
+    model = build_model(TINY, generate_state_dict(TINY, seed=2, dtype=torch.float32),
+                        dtype=torch.float32, device=DEV)
+    layer = model.model.layers[1]
+    lin = layer.self_attn.o_proj if which == "o_proj" else layer.mlp.down_proj
+    w = lin.weight.data
+    if how == "strided":
+        lin.weight = torch.nn.Parameter(w.t().contiguous().t(), requires_grad=False)
+    else:
+        flat = torch.empty(w.numel() + 1, device=DEV)
+        flat[1:] = w.flatten()
+        lin.weight = torch.nn.Parameter(flat[1:].view_as(w), requires_grad=False)
+    ids = torch.randint(0, TINY.vocab, (3, 5), generator=torch.Generator().manual_seed(1)).to(DEV)
+    rows = torch.arange(3, dtype=torch.int32, device=DEV)
+
+    def run():
+        pool = _histories(model, [5, 20, 40], 5)
+        return forward_hidden(model, ids, pool.device_kv(), rows, 45)
+
+    got = run()
+    monkeypatch.setattr(fwd_mod, "SMALL_BATCH_FUSION", False)
+    assert torch.equal(got, run())
