@@ -8,6 +8,20 @@
 
 namespace kve {
 
+// Compute units of the current device (cached per device).
+inline int resident_cus() {
+  static int cus[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cus[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+      n = 256;
+    cus[dev] = n;
+  }
+  return cus[dev];
+}
+
 // s_waitcnt immediate: at most n vector-memory operations and no LDS operation
 // of this wave outstanding (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt
 // bits 6:4 left at their maximum, lgkmcnt bits 11:8 = 0).

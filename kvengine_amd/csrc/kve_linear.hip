@@ -1700,42 +1700,35 @@ extern "C" int kve_gate_up_silu(const void* xn, const void* weight, void* act, i
   return check_launch("kve_gate_up_silu");
 }
 
-// Compute units of the current device (cached per device).
-static int resident_cus() {
-  static int cus[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cus[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    cus[dev] = n;
-  }
-  return cus[dev];
-}
-
 // Row tile of a kve_linear_rows launch. Two workgroups share a CU; a round of
 // tiles that leaves at most one per CU takes about 0.62 of a full one, and a
 // tile's fixed cost (first loads, outputs) is that of about 63 rows. Fitted to
 // gate/up, down and o at 200-6154 rows: the tile it picks was within 4 % of the
 // fastest of 128 / 160 / 192 / 256 rows at each.
 static float rows_cost(int rows, int bm, int cols) {
-  const int tiles = cdiv(rows, bm) * cols, slots = 2 * resident_cus();
-  const int rem = tiles % slots;
+  const int64_t tiles = static_cast<int64_t>(cdiv(rows, bm)) * cols, slots = 2 * resident_cus();
+  const int64_t rem = tiles % slots;
   return (tiles / slots + (rem == 0 ? 0.0f : rem <= slots / 2 ? 0.62f : 1.0f)) * (bm + 63);
 }
 
-// Slices kve_linear_rows writes: every k-slice while the partial sums' traffic
-// (written and read back) costs less than one workgroup's walk over all of K,
-// else their sum (1). Gate/up always writes its activation. 3B shapes, slices
-// and their reduction against the sum: down (K 11008) at 1024 rows 61 against
-// 74 us, at 1777 113 against 86; o (K 2048) at 400 rows 17.5 against 18.7, at
-// 700 28 against 20: the lines cross near 157 MB at K 11008 and 52 MB at 2048.
+// Slices kve_linear_rows writes: every k-slice, or their sum (1). A tile of the
+// sum walks all of K and a narrow weight has few of them; slices divide the
+// walk by S on S times the tiles, and pay for the partial sums that the
+// reduction reads back, nearly twice as much for what exceeds the L2s' 32 MB.
+// Fitted to o, q/k/v and down of both models at 165-2600 rows, projection +
+// reduction: the form it picks is within 6 % of the faster one at each, and
+// within 9 % at seven other widths (512-2048 x 512-8960). Slices / sum, us: [2048, 2048] at 500 rows 21.4 / 23.2, at 550 24.0 / 23.3;
+// [896, 896] at 500 14.6 / 14.8, at 660 17.1 / 15.4; [896, 4864] at 1600 35.1 /
+// 38.4, at 1777 42.3 / 38.4; [2048, 11008] at 1000 65.6 / 75.3, at 1200 76.7 /
+// 74.8. Gate/up always writes its activation.
 static int rows_slices(int rows, int N, int K, int mode) {
   if (mode == 2) return 1;
-  const int S = splitk_slices(N, K);
-  const int64_t traffic = int64_t{8} * S * rows * N;
-  return traffic <= 28000000 + int64_t{11700} * K ? S : 1;
+  const int S = splitk_slices(N, K), nx = N / 128;
+  const float sum = std::min(rows_cost(rows, 128, nx), rows_cost(rows, 160, nx));
+  const float slice = std::min({rows_cost(rows, 128, nx * S), rows_cost(rows, 160, nx * S),
+                                rows_cost(rows, 192, nx * S)}) / S;
+  const float mb = 4e-6f * S * rows * N;  // of partial sums
+  return 1e-3f * K * (sum - slice) > 5.8f * mb + 5.25f * std::max(0.0f, mb - 33.6f) ? S : 1;
 }
 
 extern "C" int kve_linear_rows_slices(int rows, int out_features, int in_features, int mode) {

@@ -70,3 +70,24 @@ def test_blocked_layout_is_the_documented_one():
         assert torch.equal(flat[idx], m)
         assert torch.equal(kernels.from_blocked(b, R), m)
         assert flat.abs().sum() == m.abs().sum()  # the padding rows are zeros
+
+
+def test_linear_rows_slices_see_the_width_of_the_weight():
+    """Slices or their sum, on both sides of where the measured times cross: a
+    narrow weight with a long K keeps its slices for longer than a wide one
+    with a short K."""
+    from kvengine_amd import _lib
+
+    lib = _lib.lib()
+
+    def sliced(rows, out, in_):
+        s = lib.kve_linear_rows_slices(rows, out, in_, 0)
+        assert s in (1, lib.kve_splitk_slices(out, in_))
+        return s > 1
+
+    for out, in_, last, first in ((2048, 2048, 500, 600), (2560, 2048, 350, 550), (896, 896, 500, 770),
+                                  (1152, 896, 400, 600), (896, 4864, 1600, 1777),
+                                  (2048, 11008, 1000, 1400)):
+        assert all(sliced(m, out, in_) for m in range(161, last + 1, 13)), (out, in_)
+        assert sliced(last, out, in_), (out, in_)
+        assert not any(sliced(m, out, in_) for m in (first, 2 * first, 6154)), (out, in_)
