@@ -1141,11 +1141,9 @@ __attribute__((amdgpu_waves_per_eu(NT >= 2 && NT * KW <= 6 ? 4 : 1))) void verif
 // The first two units' states are read before the item's record arrives (its
 // slots follow from its index), the next SPL together once it has, so an item
 // of up to SPL + 2 units costs two round trips; an index past the plan's split
-// items exits. SPL = 16 for launches that latency bounds; 4 for a prefill's
-// many items, which have few units each: with 16, most of a batch's loads
-// re-read the item's last unit. Per launch, with the 64-channel parts: two
-// prompts of 2304 tokens (3B) 67 -> 33 us, one of 1777 (0.5B) 13.7 -> 7.5; the
-// verify shapes' 4.3-8.7 us stay.
+// items exits (SPL: merge_batch below). Per launch, 16 channels of every row ->
+// 64-channel parts with merge_batch: two prompts of 2304 tokens (3B) 67 -> 33
+// us, one of 1777 (0.5B) 13.7 -> 7.5; the verify shapes' 4.3-8.7 us stay.
 template <int D, bool BF16, int NT, int SPL>
 __global__ __launch_bounds__(64 * NT) void verify_attn_merge_kernel(AttnArgs a) {
   using elem_t = std::conditional_t<BF16, uint16_t, float>;
@@ -1387,8 +1385,18 @@ static int launch_plan(const AttnArgs& a, const AttnCfg& p, hipStream_t st) {
   return KVE_OK;
 }
 
-// Merge workgroups from which a launch is bound by its loads (three per CU).
-constexpr long long kMergeMany = 768;
+// Units a merge workgroup loads together. Launches of few workgroups are bound
+// by their round trips: 16. From three workgroups per CU on the loads count, and
+// in a batch longer than an item's units most of them re-read its last one: 4
+// while two batches cover an item (10 units), 8 for longer histories, where 4
+// makes more round trips than the other workgroups hide. Merge of 4 / 8 / 16, us:
+// 3B, 48 x 5 rows of 4 units 5.1 / 4.6 / 5.9, 96 x 9 of 8 units 7.2 / 9.9 / 14.7,
+// 48 x 1 of 16 units 4.8 / 4.3 / 4.3, of 64 12.1 / 10.5 / 10.6; a prompt of 1777
+// tokens (7 units) 11.9 / 12.7 / 18.0, of 4000 (16) 46.1 / 47.0 / 53.9.
+static int merge_batch(long long workgroups, int max_item_units) {
+  if (workgroups < 768) return 16;
+  return max_item_units <= 10 ? 4 : 8;
+}
 
 template <int D, bool BF16, int NT, int KW>
 static int launch_attn_t(const AttnArgs& a, const AttnCfg& p, hipStream_t st, bool bs16) {
@@ -1413,9 +1421,10 @@ static int launch_attn_t(const AttnArgs& a, const AttnCfg& p, hipStream_t st, bo
   // when max_ctx allows more than one unit per history)
   if (p.max_split > 0) {
     const dim3 grid(p.max_split, a.Hkv * (D / 16));
-    const auto merge = static_cast<long long>(grid.x) * grid.y >= kMergeMany
-                           ? verify_attn_merge_kernel<D, BF16, NT, 4>
-                           : verify_attn_merge_kernel<D, BF16, NT, 16>;
+    const int spl = merge_batch(static_cast<long long>(grid.x) * grid.y, p.max_item_units);
+    const auto merge = spl == 4   ? verify_attn_merge_kernel<D, BF16, NT, 4>
+                       : spl == 8 ? verify_attn_merge_kernel<D, BF16, NT, 8>
+                                  : verify_attn_merge_kernel<D, BF16, NT, 16>;
     hipLaunchKernelGGL(merge, grid, dim3(64 * NT), 0, st, a);
   }
   return KVE_OK;

@@ -1717,10 +1717,11 @@ static float rows_cost(int rows, int bm, int cols) {
 // reduction reads back, nearly twice as much for what exceeds the L2s' 32 MB.
 // Fitted to o, q/k/v and down of both models at 165-2600 rows, projection +
 // reduction: the form it picks is within 6 % of the faster one at each, and
-// within 9 % at seven other widths (512-2048 x 512-8960). Slices / sum, us: [2048, 2048] at 500 rows 21.4 / 23.2, at 550 24.0 / 23.3;
-// [896, 896] at 500 14.6 / 14.8, at 660 17.1 / 15.4; [896, 4864] at 1600 35.1 /
-// 38.4, at 1777 42.3 / 38.4; [2048, 11008] at 1000 65.6 / 75.3, at 1200 76.7 /
-// 74.8. Gate/up always writes its activation.
+// within 9 % at seven other widths (512-2048 x 512-8960). Slices / sum, us:
+// [2048, 2048] at 500 rows 21.4 / 23.2, at 550 24.0 / 23.3; [896, 896] at 500
+// 14.6 / 14.8, at 660 17.1 / 15.4; [896, 4864] at 1600 35.1 / 38.4, at 1777
+// 42.3 / 38.4; [2048, 11008] at 1000 65.6 / 75.3, at 1200 76.7 / 74.8. Gate/up
+// always writes its activation.
 static int rows_slices(int rows, int N, int K, int mode) {
   if (mode == 2) return 1;
   const int S = splitk_slices(N, K), nx = N / 128;

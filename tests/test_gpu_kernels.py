@@ -247,6 +247,34 @@ def test_attention_fixed_order_is_batch_invariant(gpu_lib, dtype, Hq, Hkv, D, un
             assert torch.equal(x, got[0]), f"position {p}: results differ between launches"
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("Hq,D,B", [(14, 64, 96), (16, 128, 48)])
+@pytest.mark.parametrize("units", [2, 6, 7, 10, 11, 19, 27])
+def test_attention_merge_of_many_items_equals_few(gpu_lib, dtype, Hq, D, B, units):
+    """768 merge workgroups and more batch an item's units by 4 (histories of up
+    to 10 units) or 8, fewer by 16: the same bits for every item, whose own unit
+    counts run from 1 to the bound, at the edges of the batches."""
+    counts = [1 + b % units for b in range(B)]
+    ctx = [max(5, 16 * n - 3 * (b % 5)) for b, n in enumerate(counts)]
+    ctx[B // 2] = 16 * units
+    case = verify_attn_case(seed=units, num_seqs=B, ctx_lens=ctx, num_q_heads=Hq, num_kv_heads=2,
+                            head_dim=D, dtype=dtype)
+
+    def run(seqs):
+        return run_attn(case.q[seqs], *case.pool, [case.tables[b] for b in seqs],
+                        [ctx[b] for b in seqs], split_blocks=1, key_waves=1, max_ctx=16 * units,
+                        table_width=units)
+
+    many = run(list(range(B)))
+    for a in range(0, B, 16):
+        part = list(range(a, a + 16))
+        assert torch.equal(run(part), many[part])
+    few = [0, B // 2, B - 1]
+    at = [case.tables[b] for b in few], [ctx[b] for b in few]
+    ref = gather_then_attend(case.q[few], *case.pool, *at)
+    check_attn(many[few], ref, case.q[few], *case.pool, *at)
+
+
 def test_attention_plan_shared_by_layers_and_repeated(gpu_lib):
     """One plan for several layers (other K/V pools): every launch matches the
     reference; launching the same layer again gives the same bits (the merge
