@@ -22,6 +22,13 @@ inline int resident_cus() {
   return cus[dev];
 }
 
+// Rounds that `tiles` workgroups take at two per CU; a last round that leaves at
+// most one per CU takes about 0.62 of a full one.
+inline float tile_rounds(int64_t tiles) {
+  const int64_t slots = 2 * resident_cus(), rem = tiles % slots;
+  return tiles / slots + (rem == 0 ? 0.0f : rem <= slots / 2 ? 0.62f : 1.0f);
+}
+
 // s_waitcnt immediate: at most n vector-memory operations and no LDS operation
 // of this wave outstanding (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt
 // bits 6:4 left at their maximum, lgkmcnt bits 11:8 = 0).

@@ -1700,15 +1700,12 @@ extern "C" int kve_gate_up_silu(const void* xn, const void* weight, void* act, i
   return check_launch("kve_gate_up_silu");
 }
 
-// Row tile of a kve_linear_rows launch. Two workgroups share a CU; a round of
-// tiles that leaves at most one per CU takes about 0.62 of a full one, and a
-// tile's fixed cost (first loads, outputs) is that of about 63 rows. Fitted to
-// gate/up, down and o at 200-6154 rows: the tile it picks was within 4 % of the
-// fastest of 128 / 160 / 192 / 256 rows at each.
+// Row tile of a kve_linear_rows launch: a tile's fixed cost (first loads,
+// outputs) is that of about 63 rows. Fitted to gate/up, down and o at 200-6154
+// rows: the tile it picks was within 4 % of the fastest of 128 / 160 / 192 / 256
+// rows at each.
 static float rows_cost(int rows, int bm, int cols) {
-  const int64_t tiles = static_cast<int64_t>(cdiv(rows, bm)) * cols, slots = 2 * resident_cus();
-  const int64_t rem = tiles % slots;
-  return (tiles / slots + (rem == 0 ? 0.0f : rem <= slots / 2 ? 0.62f : 1.0f)) * (bm + 63);
+  return tile_rounds(static_cast<int64_t>(cdiv(rows, bm)) * cols) * (bm + 63);
 }
 
 // Slices kve_linear_rows writes: every k-slice, or their sum (1). A tile of the

@@ -366,6 +366,20 @@ static int launch_lmhead_lds(const void* hidden, int64_t hs, const void* w, int 
                   : launch_lmhead_lds_t<C, false, false>(hidden, hs, w, M, H, V, o, st);
 }
 
+// Whether 65-96 blocked rows run faster over 160 embedding rows per workgroup
+// (StepGemm) than over 64 (DmaGemm). Always where the k loop is long; up to 1024
+// columns a workgroup's fixed cost (about that of 20 embedding rows) and the
+// workgroups' last round decide, so the modelled rounds of both are compared.
+// 64 / 160 rows, 80 x 896, us: V 8000 12.6 / 14.1, 32000 16.8 / 17.9, 81920 32.1
+// / 29.3, 128256 42.6 / 44.9, 140000 47.2 / 45.5, 151936 52.5 / 49.5, 200000
+// 83.6 / 71.4; 80 x 2048: 8000 22.4 / 20.1, 128256 108.1 / 105.2. 112 rows and
+// more are 6-48 % faster on StepGemm at each.
+static bool step_pays(int H, int V) {
+  if (H > 1024) return true;
+  const int wgs = cdiv(V, 160);
+  return wgs > resident_cus() && tile_rounds(cdiv(V, 64)) >= 2.15f * tile_rounds(wgs);
+}
+
 // bf16: the LDS-staged kernel (row tiles of 16, hidden rows in passes of up to
 // 160); four waves and about 56 KB of LDS, so two workgroups share a CU.
 // Measured against eight waves with 144 KB of chunk buffers (one workgroup
@@ -392,9 +406,9 @@ static int dispatch_lmhead_bf16(int M, const void* hidden, int64_t hs, const voi
   // embedding rows make 950 workgroups, 1.86 rounds of two per CU: 128 make 2.3
   // (160 x 2048: 130-136 us) and 192 1.55 (145, and 16 registers spilled).
   if (blk) {
-    if (tiles <= 6) LM_STEP(6);
-    if (tiles <= 8) LM_STEP(8);
-    LM_STEP(10);
+    if (tiles <= 6 && step_pays(H, V)) LM_STEP(6);
+    if (tiles > 6 && tiles <= 8) LM_STEP(8);
+    if (tiles > 8) LM_STEP(10);
   }
   if (tiles <= 6) LM(6, 4, 1, 2, 56 * 1024, 1);
   LM(10, 4, 2, 2, 56 * 1024, 1);

@@ -558,12 +558,12 @@ def test_lmhead_runner_up_on_model_like_rows(gpu_lib, M, H, V):
 
 
 @pytest.mark.parametrize("M", [64, 65, 96, 97, 128, 129, 160, 161, 330])
-@pytest.mark.parametrize("H", [96, 256])
-def test_lmhead_blocked_row_tiles_equal_row_major(gpu_lib, M, H):
+@pytest.mark.parametrize("H,V", [(96, 5008), (256, 5008), (1056, 5008), (96, 81904)])
+def test_lmhead_blocked_row_tiles_equal_row_major(gpu_lib, M, H, V):
     """The blocked LM head at the edges of its row tiles, a vocabulary that is no
     multiple of its 160-row tiles and an odd count of k-steps: ids, maxima and
-    runner-up of the row-major launch, bit for bit, ties included."""
-    V = 5008
+    runner-up of the row-major launch, bit for bit, ties included. 65-96 rows
+    take the 64-row tiles at the first two shapes, the 160-row ones at the others."""
     g = torch.Generator().manual_seed(M + H)
     h = torch.randint(-2, 3, (M, H), generator=g).bfloat16().to(DEV)  # many equal logits
     w = torch.randint(-2, 3, (V, H), generator=g).bfloat16().to(DEV)
