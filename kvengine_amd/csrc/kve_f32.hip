@@ -78,7 +78,7 @@ __global__ __launch_bounds__(C::NT) void f32_splitk_kernel(const uint16_t* x, co
 }
 
 // act = silu(gate) * up: workgroup = 32 activation columns (tile rows 0..31
-// gate, 32..63 up), joined through LDS.
+// gate, 32..63 up) of 16 MT rows (blockIdx.y), joined through LDS.
 template <int MT, typename C>
 __global__ __launch_bounds__(C::NT) void f32_gate_up_kernel(const uint16_t* xn, const uint16_t* w,
                                                             float* act, int M, int H, int F) {
@@ -88,14 +88,15 @@ __global__ __launch_bounds__(C::NT) void f32_gate_up_kernel(const uint16_t* xn, 
   extern __shared__ __align__(16) uint16_t sm_f32[];
   const int tid = threadIdx.x, l = tid & 63, lr = l & 15, lg = l >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), wc = wv % G::NC, wr = wv / G::NC;
-  const int f0 = blockIdx.x * HALF;
+  const int f0 = blockIdx.x * HALF, m0 = blockIdx.y * G::XROWS, Mb = min(G::XROWS, M - m0);
   f32x4 acc[WN][MTW];
 #pragma unroll
   for (int j = 0; j < WN; ++j)
 #pragma unroll
     for (int mt = 0; mt < MTW; ++mt) acc[j][mt] = f32x4{0, 0, 0, 0};
-  G::template run<false, true>(w, [f0, F](int r) { return r < HALF ? f0 + r : F + f0 + r - HALF; }, xn,
-                               2 * H, M, 2 * H, 0, H / 16, sm_f32, acc);
+  G::template run<false, true>(w, [f0, F](int r) { return r < HALF ? f0 + r : F + f0 + r - HALF; },
+                               xn + static_cast<size_t>(m0) * 2 * H, 2 * H, Mb, 2 * H, 0, H / 16, sm_f32,
+                               acc);
   float* sy = reinterpret_cast<float*>(sm_f32);  // [16 MT][64]: gate, then up
 #pragma unroll
   for (int mt = 0; mt < MTW; ++mt)
@@ -104,7 +105,7 @@ __global__ __launch_bounds__(C::NT) void f32_gate_up_kernel(const uint16_t* xn, 
       *reinterpret_cast<f32x4*>(sy + ((MTW * wr + mt) * 16 + lr) * 64 + 16 * (WN * wc + j) + 4 * lg) =
           acc[j][mt];
   __syncthreads();
-  for (int idx = tid; idx < M * (HALF / 4); idx += C::NT) {
+  for (int idx = tid; idx < Mb * (HALF / 4); idx += C::NT) {
     const int m = idx / (HALF / 4), c = 4 * (idx % (HALF / 4));
     const f32x4 g = *reinterpret_cast<const f32x4*>(sy + m * 64 + c);
     const f32x4 u = *reinterpret_cast<const f32x4*>(sy + m * 64 + HALF + c);
@@ -112,7 +113,7 @@ __global__ __launch_bounds__(C::NT) void f32_gate_up_kernel(const uint16_t* xn, 
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       o[e] = __fmul_rn(__fdiv_rn(g[e], __fadd_rn(1.0f, expf(-g[e]))), u[e]);
-    *reinterpret_cast<f32x4*>(act + static_cast<size_t>(m) * F + f0 + c) = o;
+    *reinterpret_cast<f32x4*>(act + static_cast<size_t>(m0 + m) * F + f0 + c) = o;
   }
 }
 
@@ -238,7 +239,7 @@ static int launch_f32(K kernel, size_t& granted, dim3 grid, int threads, size_t 
   return KVE_OK;
 }
 
-// Row tiles are instantiated for 1-4, 6, 8 and 10.
+// Row tiles of the k-sliced projections are instantiated for 1-4, 6, 8 and 10.
 #define KVE_F32_ROWS(M_, CASE_)         \
   switch (cdiv(M_, 16)) {               \
     case 1: CASE_(1); break;            \
@@ -268,6 +269,30 @@ static int f32_splitk(const void* x, const void* w, float* part, int M, int N, i
   return rc;
 }
 
+// Row tiles per gate/up workgroup. All of them on F / 32 workgroups left the
+// chip half idle from about 90 rows on (0.5B: 152 workgroups), and the fp32 MFMAs
+// bound those passes; groups of rows read the weights again, from L2. The cost
+// of a workgroup is modelled as its row tiles and one more (weights, outputs),
+// and the rows are divided only for a clear gain. Pass of 2 layers in a HIP graph,
+// one group -> as picked (library GEMMs), us: 0.5B 20 x 5 rows 211 -> 191 (194),
+// 32 x 5 241 -> 221 (238); 3B 20 x 5 610 -> 556 (615), 32 x 5 738 -> 667 (665), 1
+// x 160 677 -> 608 (600); 0.5B 10 x 5 stays at 151 (two groups 154).
+static int f32_gate_tiles(int M, int F) {
+  const int tiles = cdiv(M, 16);
+  auto inst = [](int mt) { return mt <= 6 ? mt : mt <= 8 ? 8 : 10; };
+  int best = inst(tiles);
+  float least = 0.93f * tile_rounds(F / 32) * (best + 1);
+  for (int groups = 2; groups <= tiles; ++groups) {
+    const int mt = inst(cdiv(tiles, groups));
+    const float cost = tile_rounds(static_cast<int64_t>(F / 32) * cdiv(tiles, mt)) * (mt + 1);
+    if (cost < least) {
+      best = mt;
+      least = cost;
+    }
+  }
+  return best;
+}
+
 static int f32_gate_up(const void* xn, const void* w, float* act, int M, int H, int F, hipStream_t st) {
   int rc = KVE_OK;
 #define KVE_CASE(MT_)                                                                          \
@@ -276,11 +301,20 @@ static int f32_gate_up(const void* xn, const void* w, float* act, int M, int H, 
     constexpr size_t stage = static_cast<size_t>(16) * MT_ * 64 * 4;                           \
     constexpr size_t lds = C::G::LDS_BYTES > stage ? C::G::LDS_BYTES : stage;                  \
     static size_t granted_ = 0;                                                                \
-    rc = launch_f32(f32_gate_up_kernel<MT_, C>, granted_, dim3(F / 32), C::NT, lds, st,         \
+    rc = launch_f32(f32_gate_up_kernel<MT_, C>, granted_, dim3(F / 32, cdiv(M, 16 * MT_)), C::NT, lds, st, \
                     static_cast<const uint16_t*>(xn), static_cast<const uint16_t*>(w), act, M, \
                     H, F);                                                                     \
   } while (0)
-  KVE_F32_ROWS(M, KVE_CASE)
+  switch (f32_gate_tiles(M, F)) {
+    case 1: KVE_CASE(1); break;
+    case 2: KVE_CASE(2); break;
+    case 3: KVE_CASE(3); break;
+    case 4: KVE_CASE(4); break;
+    case 5: KVE_CASE(5); break;
+    case 6: KVE_CASE(6); break;
+    case 8: KVE_CASE(8); break;
+    default: KVE_CASE(10); break;
+  }
 #undef KVE_CASE
   return rc;
 }

@@ -1121,3 +1121,37 @@ def test_f32_weights_the_pass_does_not_read(gpu_lib, which, how, monkeypatch):
     got = run()
     monkeypatch.setattr(fwd_mod, "SMALL_BATCH_FUSION", False)
     assert torch.equal(got, run())
+
+
+@pytest.mark.parametrize("ffn", [4864, 16384])
+def test_f32_pass_row_tiles_and_wide_hidden(gpu_lib, ffn, monkeypatch):
+    """kve_f32_pass at every count of row tiles (3 to 10 here) on a hidden size
+    with a second, partly filled column group (1088 > 1024), histories of one
+    and of two attention units. Gate/up divides the rows over groups of
+    workgroups at ffn 4864 (1, 2 or 3 tiles each, a ragged last group) and keeps
+    them whole at 16384 (every instantiated tile). Against the library GEMMs: a sum
+    of K terms moves by about sqrt(K) 2^-24 (7.6e-6 at 16384) in either order,
+    both together stay below 2e-5 of the largest value. A sequence alone gets
+    the bits it gets in the batch."""
+    arch = dataclasses.replace(TINY, name=f"f32-{ffn}", num_layers=1, hidden=1088, ffn=ffn)
+    model = build_model(arch, generate_state_dict(arch, seed=5, dtype=torch.float32),
+                        dtype=torch.float32, device=DEV)
+    for B, T in [(11, 3), (24, 2), (32, 2), (13, 5), (16, 5), (32, 3), (33, 3), (16, 7), (32, 4),
+                 (43, 3), (16, 10)]:
+        assert fwd_mod._f32_ok(model, B * T)
+        ids = torch.randint(0, arch.vocab, (B, T), generator=torch.Generator().manual_seed(B)).to(DEV)
+        hist = [1 + 37 * b % 200 for b in range(B)]
+
+        def run(seqs, fuse):
+            monkeypatch.setattr(fwd_mod, "SMALL_BATCH_FUSION", fuse)
+            pool = _histories(model, hist, T, blocks=14)
+            rows = torch.tensor(seqs, dtype=torch.int32, device=DEV)
+            h = forward_hidden(model, ids[seqs], pool.device_kv(), rows, max(hist) + T,
+                               attn_order=(8, 1))
+            return h, pool.k, pool.v
+
+        everyone = list(range(B))
+        got = run(everyone, True)
+        for x, y in zip(got, run(everyone, False)):
+            assert (x - y).abs().max() <= 2e-5 * y.abs().max(), (B, T)
+        assert torch.equal(run([B - 1], True)[0][0], got[0][B - 1]), (B, T)
