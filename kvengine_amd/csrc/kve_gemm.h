@@ -101,12 +101,6 @@ struct DmaGemm {
   static constexpr int SWM = UPR >= 16 ? 15 : UPR - 1;
   __device__ __forceinline__ static int swz(int r) { return (r / RPS) & SWM; }
 
-  struct NoStep {
-    __device__ __forceinline__ void operator()(int) const {}
-  };
-
-  // after(ks) runs once every wave's MFMAs of k-step ks (< ks1) are issued, in
-  // k-step order: a caller can fold or restart acc there (k-slice boundaries).
   // BLK: weight and activation matrices in the blocked layout (blk_off; the
   // activation rows padded to 16, xstride unused): a chunk's 16-row tile of a
   // k-step is one contiguous 1 KB block, so an instruction reads two 512-byte
@@ -115,11 +109,10 @@ struct DmaGemm {
   // F32: fp32 matrices read as uint16 pairs (K, xstride, ks0 and ks1 count
   // uint16: a k-step is 16 values); a lane's fragments hold four consecutive k
   // of their row, multiplied by four 16x16x4 MFMAs.
-  template <bool BLK = false, bool F32 = false, typename WRow, typename After = NoStep>
+  template <bool BLK = false, bool F32 = false, typename WRow>
   __device__ __forceinline__ static void run(const uint16_t* w, WRow wrow, const uint16_t* x,
                                              int64_t xstride, int M, int K, int ks0, int ks1,
-                                             uint16_t* lds, f32x4 (&acc)[WN][MTW],
-                                             After after = After{}) {
+                                             uint16_t* lds, f32x4 (&acc)[WN][MTW]) {
     const int tid = threadIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wc = wv % NC, wr = wv / NC;
@@ -190,7 +183,6 @@ struct DmaGemm {
               acc[j][mt] = mfma16x16x32_bf16(av[j], fb[cur][mt], acc[j][mt]);
             }
           }
-        if (live) after(c0 + kk);
       }
     };
     const int nch = (ks1 - ks0 + KC - 1) / KC;
@@ -234,6 +226,8 @@ struct StepGemm {
     __device__ __forceinline__ void operator()(int) const {}
   };
 
+  // after(ks) runs once every wave's MFMAs of k-step ks are issued, in k-step
+  // order: a caller can fold or restart acc there (k-slice boundaries).
   template <bool BLK = false, typename WRow, typename After = NoStep>
   __device__ __forceinline__ static void run(const uint16_t* w, WRow wrow, const uint16_t* x,
                                              int64_t xstride, int M, int K, int ks0, int ks1,
