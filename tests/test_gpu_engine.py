@@ -6,6 +6,7 @@ requests in the documented lockstep order on the CPU. Tokens, accept traces,
 preemptions and both pools' block tables after every iteration must agree.
 """
 
+import gc
 import random
 
 import pytest
@@ -419,3 +420,29 @@ def test_graphed_prefill_writes_eager_kv(gpu_lib, bf16_models):
             seq.free()
     assert sorted(tb for _, tb in eng._pgraphs) == [64, 64, 320, 320]
     assert all(g.graph is not None for g in eng._pgraphs.values())
+
+
+def test_engine_captures_without_the_collector(gpu_lib, bf16_models, monkeypatch):
+    """Every pass of an iteration's or a prefill's capture finds automatic
+    collection off, the others find it on, and it is on again afterwards."""
+    from kvengine_amd import engine as engine_mod
+
+    seen = {}
+
+    def watch(name):
+        forward = getattr(engine_mod, name)
+
+        def watched(*a, **kw):
+            seen.setdefault(name, set()).add((torch.cuda.is_current_stream_capturing(), gc.isenabled()))
+            return forward(*a, **kw)
+
+        monkeypatch.setattr(engine_mod, name, watched)
+
+    watch("forward_hidden")
+    watch("forward_packed_wide")
+    tgt, drf = bf16_models
+    eng = SpecEngine(tgt, drf, k=3, slots=1, t_blocks=100, d_blocks=100, block_size=4, max_ctx=128)
+    eng.run([SpecRequest(i, p, 6) for i, (p, _) in enumerate(workload(3, seed=2))])
+    assert (True, False) in seen["forward_hidden"], seen
+    assert set().union(*seen.values()) <= {(False, True), (True, False)}, seen
+    assert gc.isenabled()

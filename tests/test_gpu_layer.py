@@ -900,12 +900,12 @@ def test_linear_rows_tile_edges(gpu_lib, M, N, K, mode, blocked):
 
 @pytest.mark.parametrize("n,R,C", [(1, 1, 32), (17, 40, 896), (160, 333, 2048), (33, 33, 96)])
 def test_gather_rows_and_scattered_q(gpu_lib, n, R, C):
-    """kve_gather_rows copies the indexed rows in either layout (an index outside
-    src leaves its row as it is); kve_qkv_part_rope_to with a row map writes the
-    q of kve_qkv_part_rope to the mapped rows and touches no other."""
+    """kve_gather_rows copies the indexed rows in either layout; kve_qkv_part_rope_to
+    with a row map writes the q of kve_qkv_part_rope to the mapped rows and
+    touches no other."""
     g = torch.Generator().manual_seed(n + R + C)
     src = torch.randn(R, C, generator=g).bfloat16().to(DEV)
-    idx = torch.randperm(R, generator=g)[:n].to(DEV) if n <= R else torch.zeros(n, dtype=torch.long)
+    idx = torch.randperm(R, generator=g)[:n].to(DEV)
     assert torch.equal(kernels.gather_rows(src, idx), src[idx])
     assert torch.equal(kernels.from_blocked(kernels.gather_rows(src, idx, blocked=True), n), src[idx])
     Hq, Hkv, D, bs, S = 4, 2, 64, 16, (1 if n % 2 else 3)
@@ -925,6 +925,46 @@ def test_gather_rows_and_scattered_q(gpu_lib, n, R, C):
     assert (out[rest] == 7.0).all()
     for a, b in zip(*pools):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("blocked", [False, True])
+def test_row_indices_outside_their_matrix_move_nothing(gpu_lib, blocked):
+    """kve_gather_rows leaves a row of dst whose index is not a row of src as it
+    is, and kve_qkv_part_rope_to drops a q whose row is not one of q_out, while
+    its K/V still land at their slots."""
+    n, R, C = 19, 7, 96
+    g = torch.Generator().manual_seed(n)
+    src = torch.randn(R, C, generator=g).bfloat16().to(DEV)
+    idx = torch.randint(0, R, (n,), generator=g)
+    bad = torch.tensor([0, 4, 5, 16, 18])
+    idx[bad] = torch.tensor([-1, R, 1 << 40, -(1 << 40), R + 1])
+    dst = torch.full((kernels.blocked_rows(n), C), 7.0, dtype=torch.bfloat16, device=DEV)
+    idx = idx.to(DEV)
+    rc = gpu_lib.kve_gather_rows(src.data_ptr(), idx.data_ptr(), dst.data_ptr(), n, R, C,
+                                 kernels._layout(blocked), kernels._stream(src.device))
+    assert rc == 0
+    got = kernels.from_blocked(dst, n) if blocked else dst[:n]
+    keep = torch.ones(n, dtype=torch.bool)
+    keep[bad] = False
+    assert torch.equal(got[keep], src[idx[keep]]) and (got[bad] == 7.0).all()
+    Hq, Hkv, D, bs, cap = 4, 2, 64, 16, 30
+    part = torch.randn(2, n, (Hq + 2 * Hkv) * D, generator=g).to(DEV)
+    bias = torch.randn(part.shape[2], generator=g).bfloat16().to(DEV)
+    cos, sin = (torch.randn(n, D, generator=g).bfloat16().to(DEV) for _ in range(2))
+    slots = torch.arange(n, dtype=torch.int32, device=DEV)
+    pools = [[torch.zeros(2, Hkv, *s, dtype=torch.bfloat16, device=DEV) for s in ((bs, D), (D, bs))]
+             for _ in range(2)]
+    want = kernels.qkv_part_rope(part, bias, cos, sin, slots, *pools[0], Hq, n).view(n, -1)
+    rows = torch.randperm(cap, generator=g)[:n]
+    rows[bad] = torch.tensor([-1, cap, 1 << 40, -(1 << 40), cap + 1])
+    out = torch.full((cap, Hq * D), 7.0, dtype=torch.bfloat16, device=DEV)
+    kernels.qkv_part_rope(part, bias, cos, sin, slots, *pools[1], Hq, n, q_out=out, q_rows=rows.to(DEV))
+    assert torch.equal(out[rows[keep]], want[keep])
+    rest = torch.ones(cap, dtype=torch.bool)
+    rest[rows[keep]] = False
+    assert (out[rest] == 7.0).all()
+    for x, y in zip(*pools):
+        assert torch.equal(x, y)
 
 
 @pytest.mark.parametrize("arch", [TINY, TINY128], ids=["d64", "d128"])

@@ -412,3 +412,23 @@ def test_config0_self_speculation(gpu_lib):
     assert r.acceptance_rate > 0.9
     if first is None:
         assert r.accepted_per_iter == fx["spec_self"]["accepted_per_iter"]
+
+
+def test_iterations_are_captured_without_the_collector(gpu_lib, tiny_models, monkeypatch):
+    """Every pass that runs under a capture finds automatic collection off, the
+    eager ones find it on, and it is on again after the call."""
+    from kvengine_amd import speculative as spec_mod
+
+    fx, model = tiny_models["tiny_bf16.json"]
+    seen = set()
+    forward = spec_mod.forward_hidden
+
+    def watched(*a, **kw):
+        seen.add((torch.cuda.is_current_stream_capturing(), gc.isenabled()))
+        return forward(*a, **kw)
+
+    monkeypatch.setattr(spec_mod, "forward_hidden", watched)
+    speculative_greedy(model, model, torch.tensor([fx["prompt"]], device=DEV),
+                       pool_for(model).new_sequence("t"), pool_for(model).new_sequence("d"), k=2,
+                       max_new_tokens=8, eos_token_id=None)
+    assert seen == {(False, True), (True, False)} and gc.isenabled()
