@@ -13,8 +13,8 @@
 // An fp32 matrix is read as one of uint16 pairs by DmaGemm (kve_gemm.h): its
 // k-step of 64 bytes is 16 values, and a lane's 16-byte fragment of both
 // operands is 4 consecutive k, fed to four 16x16x4 MFMAs. Every sum is fp32 in a
-// fixed order that depends on the weight's shape only, so a row's result does
-// not depend on the batch.
+// fixed order that depends on the weight's shape only, so with a fixed attention
+// order (unit_blocks, key_waves) a row's result does not depend on the batch.
 
 #include "kve_common.h"
 #include "kve_gemm.h"
@@ -274,20 +274,20 @@ static int f32_splitk(const void* x, const void* w, float* part, int M, int N, i
 // bound those passes; groups of rows read the weights again, from L2. The cost
 // of a workgroup is modelled as its row tiles and one more (weights, outputs),
 // and the rows are divided only for a clear gain. Pass of 2 layers in a HIP graph,
-// one group -> as picked (library GEMMs), us: 0.5B 20 x 5 rows 211 -> 191 (194),
-// 32 x 5 241 -> 221 (238); 3B 20 x 5 610 -> 556 (615), 32 x 5 738 -> 667 (665), 1
-// x 160 677 -> 608 (600); 0.5B 10 x 5 stays at 151 (two groups 154).
+// one group -> as picked (library GEMMs), us: 0.5B 20 x 5 rows 211 -> 193 (196),
+// 32 x 5 241 -> 214 (245); 3B 20 x 5 610 -> 559 (606), 32 x 5 738 -> 670 (666), 1
+// x 160 677 -> 615 (601); 0.5B 10 x 5 stays whole (two groups 2 % slower).
 static int f32_gate_tiles(int M, int F) {
   const int tiles = cdiv(M, 16);
-  auto inst = [](int mt) { return mt <= 6 ? mt : mt <= 8 ? 8 : 10; };
-  int best = inst(tiles);
-  float least = 0.93f * tile_rounds(F / 32) * (best + 1);
-  for (int groups = 2; groups <= tiles; ++groups) {
-    const int mt = inst(cdiv(tiles, groups));
+  int best = 0;
+  float least = 0.0f;
+  // at most 6: the four chains of more tiles leave room for one workgroup per CU
+  for (int groups = cdiv(tiles, 6); groups <= tiles; ++groups) {
+    const int mt = cdiv(tiles, groups);
     const float cost = tile_rounds(static_cast<int64_t>(F / 32) * cdiv(tiles, mt)) * (mt + 1);
-    if (cost < least) {
+    if (!best || cost < least) {
       best = mt;
-      least = cost;
+      least = groups == 1 ? 0.93f * cost : cost;
     }
   }
   return best;
@@ -311,9 +311,7 @@ static int f32_gate_up(const void* xn, const void* w, float* act, int M, int H, 
     case 3: KVE_CASE(3); break;
     case 4: KVE_CASE(4); break;
     case 5: KVE_CASE(5); break;
-    case 6: KVE_CASE(6); break;
-    case 8: KVE_CASE(8); break;
-    default: KVE_CASE(10); break;
+    default: KVE_CASE(6); break;
   }
 #undef KVE_CASE
   return rc;

@@ -13,7 +13,7 @@ import torch
 import torch.nn.functional as F
 
 from kvengine_amd import _lib, forward as fwd_mod, kernels
-from kvengine_amd.arch import TINY, TINY128
+from kvengine_amd.arch import QWEN25_0_5B, TINY, TINY128
 from kvengine_amd.decode import greedy_paged
 from kvengine_amd.forward import apply_rope, forward_hidden
 from kvengine_amd.model import RMSNorm, RotaryEmbedding, build_model
@@ -1169,7 +1169,7 @@ def test_f32_pass_row_tiles_and_wide_hidden(gpu_lib, ffn, monkeypatch):
     with a second, partly filled column group (1088 > 1024), histories of one
     and of two attention units. Gate/up divides the rows over groups of
     workgroups at ffn 4864 (1, 2 or 3 tiles each, a ragged last group) and keeps
-    them whole at 16384 (every instantiated tile). Against the library GEMMs: a sum
+    up to 6 tiles whole at 16384 (every instantiated tile; up to 96 rows there). Against the library GEMMs: a sum
     of K terms moves by about sqrt(K) 2^-24 (7.6e-6 at 16384) in either order,
     both together stay below 2e-5 of the largest value. A sequence alone gets
     the bits it gets in the batch."""
@@ -1178,7 +1178,9 @@ def test_f32_pass_row_tiles_and_wide_hidden(gpu_lib, ffn, monkeypatch):
                         dtype=torch.float32, device=DEV)
     for B, T in [(11, 3), (24, 2), (32, 2), (13, 5), (16, 5), (32, 3), (33, 3), (16, 7), (32, 4),
                  (43, 3), (16, 10)]:
-        assert fwd_mod._f32_ok(model, B * T)
+        if not fwd_mod._f32_ok(model, B * T):
+            assert ffn == 16384 and B * T > 96
+            continue
         ids = torch.randint(0, arch.vocab, (B, T), generator=torch.Generator().manual_seed(B)).to(DEV)
         hist = [1 + 37 * b % 200 for b in range(B)]
 
@@ -1195,3 +1197,50 @@ def test_f32_pass_row_tiles_and_wide_hidden(gpu_lib, ffn, monkeypatch):
         for x, y in zip(got, run(everyone, False)):
             assert (x - y).abs().max() <= 2e-5 * y.abs().max(), (B, T)
         assert torch.equal(run([B - 1], True)[0][0], got[0][B - 1]), (B, T)
+
+
+def _layer_in_64_bits(model, arch, ids):
+    """Final-normed rows of a one-layer model over a prompt, in float64 (the
+    rotary table as the model holds it)."""
+    inner, layer = model.model, model.model.layers[0]
+    a, mlp, D = layer.self_attn, layer.mlp, arch.head_dim
+
+    def rms(x, norm):
+        return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + norm.variance_epsilon) \
+            * norm.weight.double()
+
+    x = inner.embed_tokens.weight[ids].double()
+    n = len(ids)
+    q, k, v = (rms(x, layer.input_layernorm) @ a.qkv_weight.double().t() + a.qkv_bias.double()).split(
+        [arch.q_dim, arch.kv_dim, arch.kv_dim], -1)
+    cos, sin = (t[:n].double() for t in inner.rotary_emb.table(a.qkv_weight, n))
+    q, k = apply_rope(q.view(1, n, -1, D), k.view(1, n, -1, D), cos[None], sin[None], unsqueeze_dim=2)
+    v = v.view(1, n, -1, D)
+    mask = torch.ones(n, n, dtype=torch.bool, device=DEV).triu(1)
+    out = torch.empty_like(q)
+    for h in range(arch.num_q_heads):
+        g = h // arch.group
+        s = q[0, :, h] @ k[0, :, g].t().contiguous() * a.scaling
+        out[0, :, h] = torch.softmax(s.masked_fill(mask, -torch.inf), -1) @ v[0, :, g].contiguous()
+    x = x + out.view(n, -1) @ a.o_proj.weight.double().t()
+    gate, up = (rms(x, layer.post_attention_layernorm) @ mlp.gate_up_weight.double().t()).chunk(2, -1)
+    return rms(x + (F.silu(gate) * up) @ mlp.down_proj.weight.double().t(), inner.norm)
+
+
+@pytest.mark.parametrize("rows", [1, 3, 8, 15, 16, 20, 48, 65, 100, 160])
+def test_f32_pass_is_no_further_from_64_bits_than_the_library_layer(gpu_lib, rows, monkeypatch):
+    """The 2-norm error of the fp32 pass against float64, at the 0.5B's widths, is
+    at most that of the layer of library GEMMs (measured 0.37-0.90 of it)."""
+    arch = dataclasses.replace(QWEN25_0_5B, name="0.5b-l1", num_layers=1, vocab=1000)
+    model = build_model(arch, generate_state_dict(arch, seed=1, dtype=torch.float32),
+                        dtype=torch.float32, device=DEV)
+    ids = torch.randint(0, arch.vocab, (1, rows), generator=torch.Generator().manual_seed(rows)).to(DEV)
+    want = _layer_in_64_bits(model, arch, ids[0])
+    err = []
+    for fuse in (True, False):
+        monkeypatch.setattr(fwd_mod, "SMALL_BATCH_FUSION", fuse)
+        seq = PagedKVCache.for_model(model, num_blocks=12, block_size=16).new_sequence("r")
+        seq.reserve(rows)
+        h = forward_hidden(model, ids, seq.device_kv(), seq.row_dev, rows)
+        err.append(((h[0].double() - want).norm() / want.norm()).item())
+    assert err[0] <= err[1] < 1e-5, err
