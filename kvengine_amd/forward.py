@@ -569,7 +569,12 @@ def _pass_layers(model, blk: bool = False):
 
 
 def _f32_ok(model, rows: int) -> bool:
-    """kve_f32_pass takes this model's layers and this many rows."""
+    """kve_f32_pass takes this model's layers and this many rows, and is no slower
+    than the library GEMMs: from 97 rows on the fp32 MFMAs bound a pass, and on
+    ffn widths that fill the chip with whole rounds of workgroups the library's
+    tiles are the better ones (ffn 16384, hidden 1088, 2 layers in a HIP graph,
+    pass / library, us: 65 rows 344 / 360, 100 448 / 406, 160 540 / 478; the 3B's
+    11008 at 100 rows 558 / 607, at 160 670 / 666)."""
     if not SMALL_BATCH_FUSION or rows > kernels.F32_PASS_ROWS:
         return False
     layer = model.model.layers[0]
@@ -578,7 +583,7 @@ def _f32_ok(model, rows: int) -> bool:
             or mlp.down_proj.bias is not None or a.head_dim not in (64, 128):
         return False
     H, F = mlp.down_proj.weight.shape
-    return H % 64 == 0 and H <= 2048 and F % 64 == 0
+    return H % 64 == 0 and H <= 2048 and F % 64 == 0 and (rows <= 96 or F <= 12288)
 
 
 def _forward_f32(model, input_ids, kv: DeviceKV, rows, max_ctx, q_lens, attn_order):
