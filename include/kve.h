@@ -450,9 +450,9 @@ int kve_gate_up_silu(const void* xn, const void* weight, void* act, int rows, in
  *   mode 0, 1: out = fp32 partials [S, rows, out], S = kve_linear_rows_slices(...):
  *           S = 1 holds the slices' whole sum in kve_residual_norm's order
  *           (mode 0) or kve_qkv_part_rope's (mode 1); S > 1 holds every
- *           k-slice as kve_linear_splitk does (chosen when the row count is
- *           too small to fill the chip otherwise). Finish with
- *           kve_residual_norm / kve_qkv_part_rope(out, S, ...).
+ *           k-slice as kve_linear_splitk does (chosen while dividing the walk
+ *           over `in` gains more than the partial sums' traffic costs). Finish
+ *           with kve_residual_norm / kve_qkv_part_rope(out, S, ...).
  *   mode 2: weight = [gate|up] [2 ffn, in]; out [rows, ffn] bf16 =
  *           kve_gate_up_silu's act. out_features = 2 ffn.
  * layout: x and weight (and mode 2's out) all row-major or all blocked; the
@@ -461,7 +461,11 @@ int kve_gate_up_silu(const void* xn, const void* weight, void* act, int rows, in
 int kve_linear_rows(const void* x, const void* weight, void* out, int rows, int out_features,
                     int in_features, int mode, int layout, void* stream);
 
-/* Slices kve_linear_rows writes for these sizes on the current device (0: bad sizes). */
+/*
+ * Slices kve_linear_rows writes for these sizes on the current device (0: bad
+ * sizes): modelled from the rounds of its tiles on the device's compute units
+ * and the bytes of the partial sums; every kve_splitk_slices slice, or 1.
+ */
 int kve_linear_rows_slices(int rows, int out_features, int in_features, int mode);
 
 /*
@@ -493,7 +497,9 @@ int kve_small_pass(const void* const* layer_ptrs, const float* layer_consts, int
  * kve_f32_pass: every layer of an fp32 pass of at most 160 rows in one host call
  * (forward.py:187-208), the projections as k-slices whose fixed-order sums are
  * finished by bias + RoPE + K/V write, or by the residual add + RMSNorm; the
- * final-normed rows go to `out`. A row's result does not depend on the others.
+ * final-normed rows go to `out`. With unit_blocks and key_waves fixed a row's
+ * result does not depend on the others; with 0 the attention order is chosen per
+ * launch, from the number of sequences among other things. No layers: no work.
  * layer_ptrs, layer_consts: as for kve_small_pass, fp32 row-major weights.
  * residual [rows, hidden] is updated in place; xn [rows, hidden], q and attn_out
  * [rows, num_q_heads * head_dim] and act [rows, ffn] are scratch; partials:

@@ -1111,6 +1111,11 @@ __global__ __launch_bounds__(C::NT) void gate_up_silu_kernel(const uint16_t* xn,
 // down 332 -> 248 (836 -> 1118), o 78 -> 59 (664 -> 870); at 3000 rows 320 ->
 // 224, 172 -> 134, 64 -> 32. Measured beside it: a 256 x 256 tile on 8 waves
 // (gate/up 471-497 us at 6154 rows) or on 4 (484-506), one workgroup per CU.
+// Row-major operands come as 64-byte pieces of a row per k-step, half as long as
+// before: faster all the same except 3B shapes at some counts, us before -> now:
+// o at 500 rows 21.4 -> 23.9, down at 1000 75 -> 79 and at 6154 354 -> 373, q/k/v
+// at 6154 81 -> 88 (with their reductions); weights of these shapes have blocked
+// copies, which the package's passes read.
 template <int MTW, int NB>
 using RowsTile = StepGemm<2 * MTW, 4, 4, NB, 2>;
 
